@@ -3041,6 +3041,302 @@ __global__ __launch_bounds__(64 * (2 * NQW + 1), 1) void attn_decode_kernel(Attn
   }
 }
 
+// ---------------------------------------------------------------------------
+// Small calls: one launch, the key range dealt to the waves of a workgroup.
+//
+// A work item is 32 queries of one (batch, head), and wave w of its NW waves
+// takes key tiles w, w + NW, ... of 32 keys, each with its own online softmax,
+// its own LDS tiles and its own waits: no barrier between the first (Q in
+// LDS) and the last two (the waves' results merged in fp32 through LDS). What
+// bounds such a call is latency, not bytes or MFMAs: against the dual-stream
+// kernel and its merge kernel this form has one launch instead of two, no
+// partials in memory, and the tiles of 32 NW keys in flight at once (128 KB
+// per CU); against the paired kernel it has eight times the work items.
+// Per call, cold K/V, 24 heads x 128 (bf16), before -> now:
+//   83 queries x 128 keys 7.64 -> 5.5 us, x 415 keys 9.66 -> 8.6 us;
+//   300 x 512 keys 13.5 -> 9.5 us; causal 300 (16 over 8 heads) 11.1 -> 7.9
+//   us, causal 600 15.9 -> 11.9 us, causal 1000 25.2 -> 21.7 us.
+// A tile costs ~0.3 us of a CU (transfer, then S, softmax and PV in turn, two
+// waves a SIMD), so long key ranges stay with the other kernels
+// (wave_kernel_fits). Holding the next tile in registers as well (256 KB in
+// flight, 238 VGPRs) measured slower: 83 x 512 9.55 against 8.24 us.
+//
+//  - Tiles land by LDS DMA, as whole rows, with the prefill kernel's swizzles
+//    (PairLds, linear in the row bits: chunk of row RPP p + lr = the chunk of
+//    row lr, XOR a constant of the piece). At D = 128 a wave holds one tile
+//    and refills its K part as soon as the scores are computed and its V part
+//    after PV; at D = 64 it holds two.
+//  - Merge: the waves exchange (max, sum), scale their accumulators to the
+//    common maximum and 1 / sum, and write them as fp32 rows-of-four
+//    [dim / 4][query] (query slot XOR chunk: conflict-free both ways); every
+//    thread then adds one 16-byte output chunk over the waves in wave order
+//    and stores it, 64 chunks per instruction as whole rows.
+// ---------------------------------------------------------------------------
+constexpr int kWaveQ = 32;  // queries per work item of attn_wave_kernel
+constexpr int kWaveN = 32;  // keys per tile
+
+template <int D, int NW> struct WaveLds {
+  static constexpr int tile = kWaveN * D * 2;        // K or V tile, bytes
+  static constexpr int NST = D == 128 ? 1 : 2;       // tiles a wave holds
+  static constexpr int wave = NST * 2 * tile;        // [K stages][V stages] of one wave
+  static constexpr int q = NW * wave;                // Q rows, K-swizzled
+  static constexpr int ml = q + kWaveQ * D * 2;      // [NW][32] {m, l}
+  static constexpr int bytes = ml + NW * kWaveQ * 8;
+  static constexpr int part = kWaveQ * D * 4;        // one wave's fp32 result, over the tiles
+  static_assert(part <= wave, "results fit over the tiles");
+  static_assert(bytes <= 160 * 1024, "one workgroup's LDS");
+};
+
+// s_waitcnt vmcnt(n) for the few counts a wave of attn_wave_kernel waits for
+// (n is wave-uniform: pieces issued after the ones waited for).
+template <int P>
+__device__ __forceinline__ void wait_pieces(int later) {
+  if (later == 0) wait_vmcnt<0>();
+  else if (later == 1) wait_vmcnt<P>();
+  else if (later == 2) wait_vmcnt<2 * P>();
+  else wait_vmcnt<3 * P>();
+}
+
+template <int D, typename T, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void attn_wave_kernel(AttnArgs a) {
+  using W = WaveLds<D, NW>;
+  using L = PairLds<D>;
+  constexpr int KS = D / 16, DT = D / 32, RB = 2 * D;
+  constexpr int CR = D / 8;          // 16-byte chunks per row
+  constexpr int RPP = 64 / CR;       // rows per DMA piece
+  constexpr int NP = kWaveN / RPP;   // pieces per K (or V) tile
+  constexpr int NST = W::NST;
+  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+  prefetch_args(a);
+
+  const Coord it = locate(a, blockIdx.x, false, 0);
+  const int b = it.b, h = it.h;
+  const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int lane = int(threadIdx.x) & 63, g = lane >> 5, n = lane & 31;
+  const int q0 = it.qtile * kWaveQ;
+  const int qi = q0 + n;
+  const bool qvalid = qi < a.Lq;
+  const int cache_len = it.cache_len;
+  const uint32_t smem_b = lds_addr(smem);
+
+  // Q rows into LDS first (whole-row pieces; rows past Lq read as zeros).
+  const int lr = lane / CR, lx = lane % CR;  // this lane's row within a piece, physical chunk
+  {
+    const __amdgpu_buffer_rsrc_t rq =
+        make_rsrc(a.q + b * a.q_sb + int64_t(q0) * a.q_sl + h * a.q_sh, a.Lq - q0,
+                  int(a.q_sl) * 2, D);
+    for (int p = wid; p < kWaveQ / RPP; p += NW) {
+      const int r = p * RPP + lr;
+      const uint32_t o = uint32_t(r) * uint32_t(a.q_sl) * 2 + uint32_t(16 * (lx ^ L::kswz(r)));
+      dma_piece_at(rq, smem_b + W::q + p * 1024, q0 + r < a.Lq ? o : 0x80000000u);
+    }
+  }
+
+  // Key range of the work item and its tiles (cache tiles, then new-key tiles;
+  // see KvSrc).
+  const EndBounds eb = end_bounds(a, q0, min(q0 + kWaveQ, a.Lq) - 1);
+  const int kv_min = cache_len + eb.lo, kv_max = cache_len + eb.hi;
+  const int n_ct = (cache_len + kWaveN - 1) / kWaveN;
+  const int n_tiles = n_ct + (kv_max - cache_len + kWaveN - 1) / kWaveN;
+  const int nt = n_tiles > wid ? (n_tiles - wid + NW - 1) / NW : 0;  // this wave's tiles
+  const int c_ss2 = int(a.c_ss) * 2, k_sl2 = int(a.k_sl) * 2, v_sl2 = int(a.v_sl) * 2;
+  const int hk = a.kv_group == 1 ? h : h / a.kv_group;  // K/V head of this query head
+  const int64_t coff = b * a.c_sb + hk * a.c_sh;
+  const __amdgpu_buffer_rsrc_t kc = make_rsrc(a.ck ? a.ck + coff : a.q, cache_len, c_ss2, D);
+  const __amdgpu_buffer_rsrc_t vc = make_rsrc(a.cv ? a.cv + coff : a.q, cache_len, c_ss2, D);
+  const __amdgpu_buffer_rsrc_t kn =
+      make_rsrc(a.k + b * a.k_sb + hk * a.k_sh, kv_max - cache_len, k_sl2, D);
+  const __amdgpu_buffer_rsrc_t vn =
+      make_rsrc(a.v + b * a.v_sb + hk * a.v_sh, kv_max - cache_len, v_sl2, D);
+
+  // This wave's tile i (K or V) into its stage i mod NST.
+  const uint32_t kcol = uint32_t(lx ^ L::kswz(lr)), vcol = uint32_t(lx ^ (4 * L::vswz(lr)));
+  const uint32_t lds_w = smem_b + wid * W::wave;
+  auto send = [&](int i, bool is_k) __attribute__((always_inline)) {
+    const int t = wid + NW * i;
+    const bool in_cache = t < n_ct;
+    const __amdgpu_buffer_rsrc_t r = is_k ? (in_cache ? kc : kn) : (in_cache ? vc : vn);
+    const uint32_t stride = uint32_t(in_cache ? c_ss2 : (is_k ? k_sl2 : v_sl2));
+    const uint32_t row0 = uint32_t(in_cache ? t : t - n_ct) * kWaveN;
+    const uint32_t row = (row0 + uint32_t(lr)) * stride;
+    const uint32_t at =
+        lds_w + (is_k ? 0 : NST * W::tile) + (NST == 1 ? 0 : (i % NST) * W::tile);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const uint32_t ch = is_k ? kcol ^ uint32_t(L::kswz(p * RPP))
+                               : vcol ^ uint32_t(4 * L::vswz(p * RPP));
+      dma_piece_at(r, at + p * 1024, row + uint32_t(p * RPP) * stride + 16 * ch);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < NST; ++i)
+    if (i < nt) {
+      send(i, true);
+      send(i, false);
+    }
+  const int my_end = qvalid ? cache_len + visible_end(a, qi, cache_len) : 0;
+
+  // Operand addresses (PairAddr's, in this wave's stage 0).
+  uint32_t ka[KS], va[DT];
+  {
+    const int j = lane & 15, half = (lane >> 4) & 1;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) ka[s] = lds_w + n * RB + 16 * ((2 * s + g) ^ L::kswz(n));
+    const int r0 = 4 * g + (j >> 2);
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+      va[d] = lds_w + NST * W::tile + r0 * RB + 32 * half + 8 * (j & 3) + 64 * (d ^ L::vswz(r0));
+  }
+
+  // Q is in LDS once every wave's pieces of it have landed; the tiles' pieces
+  // stay in flight across this barrier.
+  wait_pieces<2 * NP>(min(nt, NST));
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  u32x4 qr[KS];
+  {
+    const uint32_t flip = a.negate_q ? 0x80008000u : 0u;  // exact sign flip of both halves
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      qr[s] = lds_read_b128_at(RowArea<D>::at(smem_b + W::q, n, 2 * s + g)) ^ flip;
+  }
+
+  f32x16 acc[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) acc[d] = f32x16{};
+  Softmax sm{-INFINITY, 0.f};
+  const float c = a.scale_log2;
+
+  for (int i = 0; i < nt; ++i) {
+    const int t = wid + NW * i;
+    const uint32_t st = NST == 1 ? 0u : uint32_t(i % NST) * W::tile;
+    const int later = min(nt - 1 - i, NST - 1);  // whole tiles in flight behind this one
+    // Scores (K pieces landed; behind them this tile's V and later tiles).
+    wait_pieces<NP>(1 + 2 * later);
+    f32x16 s = f32x16{};
+#pragma unroll
+    for (int k = 0; k < KS; ++k) s = Mfma<T>::run(lds_read_b128_at(ka[k] + st), qr[k], s);
+    const bool more = i + NST < nt;
+    if (more) {
+      // The K reads have returned (the MFMAs took them): refill the stage.
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      send(i + NST, true);
+    }
+    const bool in_cache = t < n_ct;
+    const int j0 = in_cache ? t * kWaveN : cache_len + (t - n_ct) * kWaveN;
+    const int lim = (in_cache ? cache_len - j0 : my_end - j0) - 4 * g;
+    if (in_cache ? j0 + kWaveN > cache_len : j0 + kWaveN > kv_min) {
+      int l = lim;
+      asm volatile("" : "+v"(l));
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (key_hidden(0, r, l)) s[r] = -INFINITY;
+    }
+    float tm[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+    for (int r = 0; r < 16; ++r) tm[r % 4] = fmaxf(tm[r % 4], s[r]);
+    const float m_new =
+        fmaxf(sm.m, xor32_max(fmaxf(fmaxf(tm[0], tm[1]), fmaxf(tm[2], tm[3]))));
+    // The reference follows the maximum exactly (softmax_max lets it lag by up
+    // to 2^8): a wave sees few tiles, and with it the largest probability of
+    // each wave's keys is 1, which 16 bits hold exactly. Error against 64 bits
+    // at 83 x 512 keys: 2.06e-3, against 2.19e-3 with the lagging reference
+    // (and 2.11e-3 from the dual-stream kernel), for 2 to 4% of the call.
+    if (__any(m_new > sm.m)) {
+      if (!__all(sm.m == -INFINITY)) {
+        const float corr = sm.m == -INFINITY ? 0.f : fast_exp2((sm.m - m_new) * c);
+        sm.l *= corr;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) acc[d] *= corr;
+      }
+      sm.m = m_new;
+    }
+    const float mb = sm.m == -INFINITY ? 0.f : sm.m * c;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = fast_exp2(__builtin_fmaf(s[r], c, -mb));
+    u32x4 pk[2];
+    float part[2] = {0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t p = Mfma<T>::pack(s[8 * u + 2 * e], s[8 * u + 2 * e + 1]);
+        pk[u][e] = p;
+        part[e & 1] = Mfma<T>::sum2(p, part[e & 1]);
+      }
+    sm.l += part[0] + part[1];
+    // PV (V pieces landed; behind them later tiles and the refilled K).
+    wait_pieces<NP>(2 * later + (more ? 1 : 0));
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+        const uint32_t vu = va[d] + st + 16 * u * RB;
+        const u32x2 lo = lds_read_tr16_at(vu);
+        const u32x2 hi = lds_read_tr16_at(vu + 8 * RB);
+        acc[d] = Mfma<T>::run(u32x4{lo[0], lo[1], hi[0], hi[1]}, pk[u], acc[d]);
+      }
+    if (more) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      send(i + NST, false);
+    }
+  }
+
+  // Merge over the waves that had tiles (at least wave 0, whose empty result
+  // makes a query with no visible key NaN: 0 * inf, as the reference).
+  const int used = min(NW, max(n_tiles, 1));
+  const float l_own = xor32_sum(sm.l);
+  const float m_own = sm.m == -INFINITY ? -INFINITY : sm.m * c;
+  f32x2* const ml = reinterpret_cast<f32x2*>(reinterpret_cast<char*>(smem) + W::ml);
+  if (g == 0) ml[wid * kWaveQ + n] = f32x2{m_own, l_own};
+  __syncthreads();  // every wave's tile reads and DMA pieces are done too
+  if (wid < used) {
+    float mm = -INFINITY;
+    f32x2 o[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      o[w] = w < used ? ml[w * kWaveQ + n] : f32x2{-INFINITY, 0.f};
+      mm = fmaxf(mm, o[w][0]);
+    }
+    const float base = mm == -INFINITY ? 0.f : mm;
+    float l_tot = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) l_tot += fast_exp2(o[w][0] - base) * o[w][1];
+    const float k = fast_exp2(m_own - base) * (1.0f / l_tot);
+    // Rows of four dims: row d4 = 8 d + 2 r4 + g holds the 32 queries, query q
+    // at slot q ^ f(d4 / 2).
+    f32x4* const mine = reinterpret_cast<f32x4*>(reinterpret_cast<char*>(smem) + wid * W::part);
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        const int d4 = 8 * d + 2 * r4 + g, ch = 4 * d + r4;
+        mine[d4 * kWaveQ + (n ^ (D == 128 ? ch : 2 * ch))] =
+            f32x4{acc[d][4 * r4] * k, acc[d][4 * r4 + 1] * k, acc[d][4 * r4 + 2] * k,
+                  acc[d][4 * r4 + 3] * k};
+      }
+  }
+  __syncthreads();
+  const f32x4* const all = reinterpret_cast<const f32x4*>(smem);
+#pragma unroll
+  for (int x = int(threadIdx.x); x < kWaveQ * CR; x += 64 * NW) {
+    const int row = x / CR, ch = x % CR;
+    const int slot = row ^ (D == 128 ? ch : 2 * ch);
+    f32x4 lo = f32x4{}, hi = f32x4{};
+    for (int w = 0; w < used; ++w) {
+      lo += all[w * (W::part / 16) + (2 * ch) * kWaveQ + slot];
+      hi += all[w * (W::part / 16) + (2 * ch + 1) * kWaveQ + slot];
+    }
+    if (q0 + row < a.Lq) {
+      const u32x4 v = {Mfma<T>::pack(lo[0], lo[1]), Mfma<T>::pack(lo[2], lo[3]),
+                       Mfma<T>::pack(hi[0], hi[1]), Mfma<T>::pack(hi[2], hi[3])};
+      *reinterpret_cast<u32x4*>(a.out + b * a.o_sb + int64_t(q0 + row) * a.o_sl + h * a.o_sh +
+                                8 * ch) = v;
+    }
+  }
+}
+
 // One wave per merge block: at C1 (83 rows x 24 heads, 8 splits) 1,056 blocks
 // of 64 threads took 12.58 us per call against 12.79 us for 264 of 256 threads
 // (13.04 and 13.98 us for 512 and 1,024 threads).
@@ -3159,13 +3455,13 @@ int device_cus() {
 }
 
 // Attention kernels a plan can pick (the DX_TUNE_ATTN_KERNEL values).
-enum AttnKernel { kSingle = 1, kDual = 2, kPaired = 3, kDecode = 4 };
+enum AttnKernel { kSingle = 1, kDual = 2, kPaired = 3, kDecode = 4, kWave = 5 };
 
 struct Plan {
   int n_qtiles;
   int bm;                    // queries per work item (decode: query-group rows)
   int kernel;                // AttnKernel
-  int nqw;                   // decode: compute waves per workgroup (2 or 3)
+  int nqw;                   // waves per workgroup: decode compute waves (2 or 3), wave kernel (4 or 8)
   int prow;                  // rows per partial in the workspace (decode: 32 per compute block)
   int n_seg;                 // 0 = uniform
   int uniform_splits;
@@ -3452,6 +3748,73 @@ Plan make_plan(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_t 
   return p;
 }
 
+// Whether a call goes to attn_wave_kernel, by its work items I (32 queries of
+// a head) and the mean key tiles T of 32 an item visits (causal and blocks: an
+// item sees about half of the new keys' tiles).
+//  - I up to one per CU (8 waves): T up to 14, or 18 from 96 items on (fewer
+//    items leave most of the chip's HBM rate unused); 18 at D = 64, whose
+//    tiles are half as long. Cold K/V, us per call, the other kernels ->
+//    this one: D 128, 24 heads, 83 x 415 9.7 -> 8.6, 83 x 512 10.0 -> 10.0,
+//    83 x 640 10.3 -> 11.0; 200 x 512 11.3 -> 9.9, 200 x 640 12.5 -> 10.9;
+//    D 64, 83 x 512 8.0 -> 7.0, 83 x 1024 8.6 -> 10.2.
+//  - More items (4 waves, two workgroups per CU): up to two per CU and T up
+//    to 20 (24 heads, 400 x 640 15.0 -> 13.3; 40 heads, 300 x 768 keys 16.9 ->
+//    15.7, but 200 x 768 14.6 -> 15.3; three items per CU: 1000 x 256 13.4 ->
+//    14.2). Under a causal or block mask of nb > 1 blocks, where the paired
+//    kernel's 256-query items see far more keys than their queries need: up
+//    to 64 (1 - 1/nb) tiles per CU at D 128 (causal 1000 25.2 -> 21.5; 16
+//    heads, causal 1400 26.6 -> 22.5, 2000 36.4 -> 37.8), 96 at D 64 (24
+//    heads, causal 1400 28.6 -> 22.2; 40 heads, 1400 29.8 -> 33.3).
+bool wave_kernel_fits(double items, double tiles, int64_t D, int64_t nb, bool causal, int cus) {
+  const double t = tiles / items;
+  if (items <= cus) return t <= (D == 64 || items * 8 >= 3 * cus ? 18 : 14);
+  if (items <= 2 * cus && t <= 20) return true;
+  const double masked = causal ? 1.0 : nb > 1 ? 1.0 - 1.0 / double(nb) : 0.0;
+  return tiles / cus <= (D == 64 ? 96 : 64) * masked;
+}
+
+// Turn the plan of a call that wave_kernel_fits into one launch of
+// attn_wave_kernel. The workspace the call has to bring is unchanged (the
+// workspace query knows no mask); this kernel leaves it untouched.
+void use_wave_kernel(Plan& p, int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D,
+                     int64_t cache_len, int64_t n_blocks, bool causal) {
+  const int forced = tuning(DX_TUNE_ATTN_KERNEL);
+  if (forced ? forced != kWave
+             : tuning(DX_TUNE_ATTN_SPLITS) != 0 || tuning(DX_TUNE_ATTN_PMERGE) != 0)
+    return;
+  const int cus = device_cus();
+  const int64_t n_qtiles = cdiv(Lq, kWaveQ), items = B * H * n_qtiles;
+  double seen = double(cdiv(Lk, kWaveN));  // mean new-key tiles of an item
+  if (causal) seen = (seen + 1) / 2;
+  else if (n_blocks > 1) seen *= double(n_blocks + 1) / double(2 * n_blocks);
+  double tiles = 0;
+  if (p.n_seg == 0) {
+    tiles = double(items) * (double(cdiv(cache_len, kWaveN)) + seen);
+  } else {
+    // A ragged batch: the longest sequence's items have to fit by themselves.
+    int64_t longest = 0;
+    for (int c : p.seg_cache) {
+      longest = std::max<int64_t>(longest, cdiv(c, kWaveN));
+      tiles += double(H * n_qtiles) * (double(cdiv(c, kWaveN)) + seen);
+    }
+    if (!forced && double(longest) + seen > 20) return;
+  }
+  if (items >= (int64_t(1) << 31)) return;  // past the grid's limit
+  if (!forced && !wave_kernel_fits(double(items), tiles, D, n_blocks, causal, cus)) return;
+  p.kernel = kWave;
+  p.nqw = items <= cus ? 8 : 4;
+  p.bm = kWaveQ;
+  p.n_qtiles = int(n_qtiles);
+  p.items = items;
+  p.uniform_splits = 1;
+  for (size_t k = 0; k < p.seg_splits.size(); ++k) {
+    p.seg_splits[k] = 1;
+    p.seg_base[k + 1] = int(int64_t(k + 1) * H * n_qtiles);
+  }
+  p.partials = p.comb_blocks = p.counter_bytes = p.ws_bytes = 0;
+  p.pmerge = p.spread = false;
+}
+
 // Opt a kernel into `bytes` of dynamic LDS (beyond the 64 KB default window;
 // gfx950 allows 160 KB per workgroup) on the current device, once per kernel
 // and device: each device holds its own copy of the kernel and its attributes.
@@ -3500,8 +3863,20 @@ hipError_t launch_decode(const AttnArgs& a, int64_t items, hipStream_t st) {
   return hipGetLastError();
 }
 
+template <int D, typename T, int NW>
+hipError_t launch_wave(const AttnArgs& a, int64_t items, hipStream_t st) {
+  constexpr int lds = WaveLds<D, NW>::bytes;
+  const hipError_t attr =
+      opt_in_lds(reinterpret_cast<const void*>(&attn_wave_kernel<D, T, NW>), lds);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL((attn_wave_kernel<D, T, NW>), dim3(unsigned(items)), dim3(64 * NW), lds, st, a);
+  return hipGetLastError();
+}
+
 template <int D, typename T>
 hipError_t launch_d(const AttnArgs& a, const Plan& p, hipStream_t st) {
+  if (p.kernel == kWave)
+    return p.nqw == 8 ? launch_wave<D, T, 8>(a, p.items, st) : launch_wave<D, T, 4>(a, p.items, st);
   hipError_t e = p.kernel == kDecode
                      ? (p.nqw == 3 ? launch_decode<D, T, 3>(a, p.items, st)
                                    : launch_decode<D, T, 2>(a, p.items, st))
@@ -3688,6 +4063,7 @@ int attention_entry(const void* q, int64_t q_sb, int64_t q_sl, int64_t q_sh, con
     }
     DX_CHECK_ARG(al16(workspace), "attention: workspace must be 16-byte aligned");
   }
+  if (!general) use_wave_kernel(p, B, Lq, Lk, H, D, cache_len, n_blocks, causal != 0);
   if (general) {
     AttnArgs a{};
     a.q = static_cast<const uint16_t*>(q); a.q_sb = q_sb; a.q_sl = q_sl; a.q_sh = q_sh;

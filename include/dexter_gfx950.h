@@ -86,7 +86,7 @@ int dx_abi_version(void);
  *   DX_TUNE_ATTN_SPLITS  key splits per attention work item (1..16)
  *   DX_TUNE_ATTN_KERNEL  attention kernel: 1 single-stream, 2 dual-stream
  *                        with a separate merge kernel, 3 paired prefill,
- *                        4 one-launch decode
+ *                        4 one-launch decode, 5 wave-split (small calls)
  *   DX_TUNE_NORM_WAVES   waves per row of the adaLN / gated-residual kernels (1..16)
  *   DX_TUNE_QKV_SPLITS   K splits of the fused QKV GEMM (1..16)
  *   DX_TUNE_QKV_WAVES    fused QKV GEMM form: 0 the LDS-DMA form (waves of 64
