@@ -3815,22 +3815,6 @@ void use_wave_kernel(Plan& p, int64_t B, int64_t Lq, int64_t Lk, int64_t H, int6
   p.pmerge = p.spread = false;
 }
 
-// Opt a kernel into `bytes` of dynamic LDS (beyond the 64 KB default window;
-// gfx950 allows 160 KB per workgroup) on the current device, once per kernel
-// and device: each device holds its own copy of the kernel and its attributes.
-hipError_t opt_in_lds(const void* fn, int bytes) {
-  static std::mutex mu;
-  static std::set<std::pair<const void*, int>> done;
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  std::lock_guard<std::mutex> lk(mu);
-  if (done.count({fn, dev})) return hipSuccess;
-  e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e == hipSuccess) done.insert({fn, dev});
-  return e;
-}
-
 template <int D, typename T, int NS>
 hipError_t launch_main(const AttnArgs& a, int64_t items, hipStream_t st) {
   constexpr int lds = NS * Lds<D>::bytes;  // double-buffered tiles per stream

@@ -6,6 +6,9 @@
 #include <stdio.h>
 
 #include <atomic>
+#include <mutex>
+#include <set>
+#include <utility>
 
 namespace dx {
 
@@ -24,6 +27,21 @@ void set_error(const char* fmt, ...) {
   va_start(ap, fmt);
   vsnprintf(g_error, sizeof(g_error), fmt, ap);
   va_end(ap);
+}
+
+// Once per kernel and device: each device holds its own copy of the kernel and
+// its attributes.
+hipError_t opt_in_lds(const void* fn, int bytes) {
+  static std::mutex mu;
+  static std::set<std::pair<const void*, int>> done;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> lk(mu);
+  if (done.count({fn, dev})) return hipSuccess;
+  e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e == hipSuccess) done.insert({fn, dev});
+  return e;
 }
 
 }  // namespace dx

@@ -125,6 +125,9 @@ namespace dx {
 void set_error(const char* fmt, ...);
 // Current value of a dx_set_tuning override (0: the library's own choice).
 int tuning(int key);
+// Opt a kernel into `bytes` of dynamic LDS (beyond the 64 KB default window;
+// gfx950 allows 160 KB per workgroup) on the current device.
+hipError_t opt_in_lds(const void* fn, int bytes);
 // Argument checks of the QK-norm + rotary prologue (qk_norm_rope.hip), also
 // run by the attention launch that does the prologue itself.
 int rope_validate(const void* q, int64_t q_sb, int64_t q_sl, int64_t q_sh,

@@ -14,6 +14,10 @@ and calls it, exactly as dexter's dispatchers do (``python/dexter/ops/__init__.p
   (no dispatcher in the reference: ``SelfAttention.forward`` runs three
   ``nn.Linear`` and ``ops.qk_norm_rope``, ``models/dreamzero/model.py:162-175``;
   here one call for decode chunks)
+* ``linear_chunk``               -> ``select("gemm", "linear_chunk", x, weight, bias)``
+  (no dispatcher in the reference: ``SelfAttention.forward``'s output projection
+  is an ``nn.Linear``, ``models/dreamzero/model.py:183``; here one kernel for
+  decode chunks)
 * ``qk_norm_rope_attention``     -> ``select("attention", "qk_norm_rope_blockwise_causal", q, k, v)``
   (no dispatcher in the reference: ``SelfAttention.forward`` calls
   ``ops.qk_norm_rope``, ``KVCache.append`` and ``ops.blockwise_causal_attention``,
@@ -36,7 +40,8 @@ from ..registry import select
 
 __all__ = ["qk_norm_rope", "blockwise_causal_attention", "kv_cache_append",
            "qk_norm_rope_append", "blockwise_causal_attention_varlen",
-           "adaln_modulate", "gated_residual", "qkv_norm_rope", "qk_norm_rope_attention"]
+           "adaln_modulate", "gated_residual", "qkv_norm_rope", "qk_norm_rope_attention",
+           "linear_chunk"]
 
 
 def qkv_norm_rope(
@@ -65,6 +70,13 @@ def qkv_norm_rope(
     return select("rope", "qkv_norm_rope", x, wq, bq, wk, bk, wv, bv, q_weight, k_weight, cos,
                   sin, heads)(x, wq, bq, wk, bk, wv, bv, q_weight, k_weight, cos, sin, heads,
                               eps, interleaved, cache, start, status)
+
+
+def linear_chunk(x: torch.Tensor, weight: torch.Tensor,
+                 bias: torch.Tensor | None = None) -> torch.Tensor:
+    """``F.linear(x, weight, bias)`` of a ``[B, L, C]`` decode chunk (at most 128 tokens,
+    ``C`` a multiple of 512, out features of 16), bf16 or f16, rounded once."""
+    return select("gemm", "linear_chunk", x, weight, bias)(x, weight, bias)
 
 
 def adaln_modulate(

@@ -16,7 +16,7 @@ import torch
 
 LIB_NAME = "libdexter_gfx950.so"
 LIB_PATH = Path(__file__).resolve().parents[2] / LIB_NAME
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 DX_OK, DX_EINVAL, DX_ELAUNCH, DX_EFULL, DX_EWORKSPACE = 0, 1, 2, 3, 4
 DX_BF16, DX_F16, DX_F32, DX_I32, DX_I64 = 0, 1, 2, 3, 4
@@ -152,6 +152,10 @@ _SIGNATURES: dict[str, tuple[type, list]] = {
         _f, _i,                    # eps, interleaved
         _p, _l, _p]),              # workspace, bytes, stream
     "dx_qkv_workspace_bytes": (_l, [_l, _l, _l, _l, _l]),
+    "dx_linear_chunk": (_i, [
+        _p, _l, _l, _i,            # x, sb, sl, io dtype
+        _p, _l, _p, _p,            # w, row stride, bias (may be null), y
+        _l, _l, _l, _l, _p]),      # B, L, C, N, stream
     "dx_adaln_modulate": (_i, [
         _p, _l, _l, _i,            # x, sb, sl, x dtype
         _p, _l, _l,                # scale, sb, sl

@@ -14,6 +14,10 @@ activations. The HIP path is a split-K MFMA GEMM that reads each weight byte
 once from every CU, then the prologue kernel summing its fp32 partials, so
 the q/k/v projections never make a bf16 round trip through HBM before the
 norm. ``start`` may be a device cursor, as for ``qk_norm_rope_append``.
+
+``linear_chunk`` (``gemm/linear_chunk``, HIP ``dx_linear_chunk``) is one
+``nn.Linear`` of a decode chunk: ``SelfAttention.forward``'s output projection
+(``models/dreamzero/model.py:183``).
 """
 
 from __future__ import annotations
@@ -22,7 +26,7 @@ import torch
 
 from ...registry import Priority, register
 from . import _lib
-from ._common import CDNA4, MATRIX_DTYPES, device_cursor, rows_ok
+from ._common import CDNA4, MATRIX_DTYPES, device_cursor, rows_ok, strides
 
 _TABLE_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 MAX_TOKENS = 128
@@ -113,3 +117,28 @@ def qkv_norm_rope(x, wq, bq, wk, bk, wv, bv, q_weight, k_weight, cos, sin, heads
         ws.data_ptr(), ws.numel(), _lib.stream_handle(x.device))
     _lib.check(rc, "qkv_norm_rope")
     return q_out, k_out, v_out
+
+
+def _accepts_linear(x, w, b) -> bool:
+    if not (x.is_cuda and x.dtype in MATRIX_DTYPES and x.dim() == 3 and w.dim() == 2):
+        return False
+    n, c = w.shape
+    return (0 < x.shape[0] * x.shape[1] <= MAX_TOKENS and x.shape[2] == c and c % 512 == 0
+            and n % 16 == 0 and _weight_ok(w, n, c, x.dtype) and w.device == x.device
+            and (b is None or (b.shape == (n,) and b.dtype == x.dtype and b.device == x.device)))
+
+
+@register("gemm", "linear_chunk", name="hip_linear_chunk_gfx950",
+          capability=CDNA4, priority=Priority.SPECIALISED, accepts=_accepts_linear)
+def linear_chunk(x, w, b):
+    bsz, seq, c = x.shape
+    if not rows_ok(x) or min(x.stride()) < 0:
+        x = x.contiguous()
+    if b is not None and (b.stride(0) != 1 or b.data_ptr() % 16):
+        b = b.clone(memory_format=torch.contiguous_format)
+    y = torch.empty((bsz, seq, w.shape[0]), device=x.device, dtype=x.dtype)
+    rc = _lib.load().dx_linear_chunk(
+        x.data_ptr(), *strides(x, 2), _lib.dtype_code(x.dtype), w.data_ptr(), w.stride(0),
+        _lib.ptr(b), y.data_ptr(), bsz, seq, c, w.shape[0], _lib.stream_handle(x.device))
+    _lib.check(rc, "linear_chunk")
+    return y

@@ -30,6 +30,9 @@
  *                            nn.Linear calls; on gfx1151 hipBLASLt through
  *                            ops/gfx1151/gemm) fused with dx_qk_norm_rope(_append)
  *                            (model.py:166-175)
+ *   dx_linear_chunk          the output projection of SelfAttention.forward
+ *                            (models/dreamzero/model.py:183, one nn.Linear;
+ *                            on gfx1151 hipBLASLt through ops/gfx1151/gemm)
  *   dx_adaln_modulate        ops/gfx1151/norm/adaln.py:108-128 (kernel :20-48;
  *                            semantics ops/reference/norm.py:16-20, dispatcher
  *                            ops/__init__.py:39-49)
@@ -76,7 +79,7 @@ const char* dx_last_error(void);
 
 /* ABI revision of this header; the Python loader checks it. */
 int dx_abi_version(void);
-#define DX_ABI_VERSION 10
+#define DX_ABI_VERSION 11
 
 /*
  * Launch-schedule overrides, for measurement and tests only: process-wide,
@@ -391,6 +394,19 @@ int dx_qkv_norm_rope(const void* x, int64_t x_sb, int64_t x_sl, int io_dtype,
 
 /* Workspace bytes dx_qkv_norm_rope needs for this shape; negative DX_E* on a bad shape. */
 int64_t dx_qkv_workspace_bytes(int64_t B, int64_t L, int64_t C, int64_t H, int64_t D);
+
+/*
+ * y = x w^T + bias of a decode chunk (nn.Linear: an fp32 sum, rounded once to
+ * io_dtype). x is [B, L, C] (strides x_sb, x_sl; C contiguous), w [N, C] (row
+ * stride w_row), bias [N] or NULL, y contiguous [B, L, N]. io_dtype: DX_BF16 or
+ * DX_F16. Limits: B*L <= 128 tokens, C a multiple of 512, N of 16, x spanning
+ * less than 2^31 bytes, w_row below 2^22 elements; pointers 16-byte aligned,
+ * strides multiples of 8 elements. No workspace.
+ * Replaces: models/dreamzero/model.py:183 (SelfAttention's output projection).
+ */
+int dx_linear_chunk(const void* x, int64_t x_sb, int64_t x_sl, int io_dtype, const void* w,
+                    int64_t w_row, const void* bias, void* y, int64_t B, int64_t L, int64_t C,
+                    int64_t N, void* stream);
 
 /*
  * Adaptive LayerNorm modulation of a [B, L, C] activation:

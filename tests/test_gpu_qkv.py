@@ -234,3 +234,41 @@ def test_self_attention_fused_projection_matches_unfused(device, built_lib, writ
     if write:
         assert_parity_scaled(caches[0].cache[0][:, :, 83:166], caches[1].cache[0][:, :, 83:166].float(),
                              what="appended rows")
+
+
+@pytest.mark.parametrize("b,l,c,n,dtype,bias", [
+    (1, 1, 512, 16, DT, True), (1, 16, 512, 48, DT, False), (1, 33, 1024, 4096, torch.float16, True),
+    (2, 32, 1536, 1536, DT, True), (1, 65, 1024, 128, DT, True), (1, 83, 3072, 3072, DT, True),
+    (4, 24, 2560, 2576, DT, False), (1, 128, 4096, 4096, torch.float16, True),
+    (1, 113, 512, 8208, DT, True),  # token tiles and feature tiles both end mid-group
+])
+def test_linear_chunk(device, built_lib, b, l, c, n, dtype, bias):
+    """``F.linear`` of a chunk, one rounding of the exact sum: within one ulp of the 64-bit
+    result plus the fp32 accumulation error, 2^-18 of the sum of |x w| (as ``v`` above)."""
+    g = torch.Generator().manual_seed(b * l + n)
+    wide = torch.randn(b, l, c + 64, generator=g).to(dtype)
+    w = (torch.randn(n, c, generator=g) * c ** -0.5).to(dtype)
+    bb = torch.randn(n, generator=g).mul(0.1).to(dtype) if bias else None
+    x = wide.to(device)[..., :c]  # rows with a stride of their own
+    wd, bd = w.to(device), None if bb is None else bb.to(device)
+    got = ops.linear_chunk(x, wd, bd)
+    assert got.shape == (b, l, n) and got.dtype == dtype
+    assert torch.equal(got, ops.linear_chunk(x, wd, bd))
+    ref = x.cpu().double() @ w.double().t() + (0 if bb is None else bb.double())
+    mag = x.cpu().double().abs() @ w.double().abs().t()
+    fi = torch.finfo(dtype)
+    ulp = torch.exp2(torch.floor(torch.log2(ref.abs().clamp_min(fi.tiny)))) * fi.eps
+    bad = (got.cpu().double() - ref).abs() > ulp + 2.0 ** -18 * mag
+    assert not bad.any(), f"{int(bad.sum())} elements beyond one ulp"
+
+
+def test_output_projection_falls_back(device, built_lib):
+    """A weight layout the chunk GEMM does not take still projects (``F.linear``)."""
+    from dexter_amd.models import SelfAttention
+    layer = SelfAttention(512, 4, dtype=DT, device=device)
+    x = torch.randn(1, 20, 512, device=device).to(DT)
+    cos, sin = (t.to(device) for t in rope_table(torch.arange(20), 128))
+    plain = layer(x, cos, sin, None, 0)
+    wt = layer.o.weight.data.t().contiguous()
+    layer.o.weight.data = wt.t()  # column-major
+    assert_parity_scaled(layer(x, cos, sin, None, 0), plain.float())
