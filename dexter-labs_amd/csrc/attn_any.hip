@@ -35,7 +35,7 @@
 // range; each split writes its unnormalised fp32 partial (acc, with the max
 // m and sum l it is relative to) after the workspace's counter region (which
 // it never writes), and a merge kernel combines the splits of each row.
-#include "attn_common.h"
+#include "attn_tile.h"
 
 #include <math.h>
 
@@ -109,46 +109,6 @@ __device__ __forceinline__ float quad_sum(float x) {
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// Cached rows of sequence b (the device cursor clamped to the capacity the
-// launch was planned for, or the per-sequence length of a ragged batch).
-__device__ __forceinline__ int any_cache_len(const AttnArgs& a, int b) {
-  if (a.cache_len_dev) return min(max(*a.cache_len_dev, 0), a.cache_len);
-  return a.n_seg ? a.seg_cache[b] : a.cache_len;
-}
-
-// Work item i of the grid. Workgroup i runs on XCD i % 8 (each XCD has its own
-// L2): with a multiple of 8 (batch, head) pairs, XCD x takes a contiguous run
-// of them, so a head's K/V (and a K/V head's query heads) go through one L2.
-// Late query tiles, which see the most keys under a causal or block mask, go
-// first. Partials stay numbered by (b, h, query tile, split). Cold, us per
-// call, before (split fastest, then query tiles in order) -> now: D 256 causal
-// 4000, 16 over 4 heads 467 -> 315; D 32 causal 4096 155 -> 91; D 256, 40 heads
-// x 1500 in blocks of 200 198 -> 153; 2048 unmasked 166 -> 159.
-struct AnyItem {
-  int b, h, qt, split;
-  int64_t partial;
-};
-__device__ __forceinline__ AnyItem any_item(const AttnArgs& a, int i) {
-  const uint32_t G = uint32_t(a.B) * uint32_t(a.H), S = uint32_t(a.n_splits);
-  uint32_t grp, rank;  // (batch, head) pair; rank within it
-  if (G % 8 == 0) {
-    const uint32_t g8 = G / 8, slot = uint32_t(i) / 8;
-    rank = slot / g8;
-    grp = uint32_t(i) % 8 * g8 + (slot - rank * g8);
-  } else {
-    rank = uint32_t(i) / G;
-    grp = uint32_t(i) - rank * G;
-  }
-  AnyItem it;
-  const uint32_t rq = rank / S;
-  it.split = int(rank - rq * S);
-  it.qt = a.n_qtiles - 1 - int(rq);
-  it.b = int(grp / uint32_t(a.H));
-  it.h = int(grp) - it.b * a.H;
-  it.partial = (int64_t(grp) * a.n_qtiles + it.qt) * S + it.split;
-  return it;
 }
 
 template <int D> struct AnyLds {

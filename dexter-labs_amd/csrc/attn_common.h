@@ -203,4 +203,11 @@ AnyPlan plan_any(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_
 // n_seg == B > 0. dtype: DX_BF16, DX_F16 or DX_F32.
 hipError_t launch_any(const AttnArgs& a, int dtype, int D, const AnyPlan& p, hipStream_t st);
 
+// Head dim 256, 16-bit inputs, one launch without key splits (attn_wide.hip);
+// a as for launch_any. wide_fits: whether it is the faster one for sequences
+// with these cache lengths.
+bool wide_fits(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t cache_len,
+               const int64_t* cache_lens, int64_t n_blocks, bool causal, int cus);
+hipError_t launch_wide(AttnArgs a, int dtype, hipStream_t st);
+
 }  // namespace dx

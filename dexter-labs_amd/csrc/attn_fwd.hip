@@ -53,7 +53,7 @@
 // on one XCD (item i runs on XCD i % 8), so its K/V and partials stay in one
 // L2. Ragged batches (one cache length per sequence) get one segment per
 // sequence with its own split count, longest sequence first.
-#include "attn_common.h"
+#include "attn_tile.h"
 
 #include <float.h>
 #include <limits.h>
@@ -107,44 +107,6 @@ constexpr int kBM = 32 * kNW;  // queries per workgroup
 constexpr int kPairWaves = 8;  // waves per workgroup of the paired-group kernel
 constexpr int kBMPair = 256;   // its queries per workgroup
 
-template <typename T> struct Mfma;
-template <> struct Mfma<bf16_t> {
-  static __device__ __forceinline__ f32x16 run(u32x4 a, u32x4 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint32_t pack(float lo, float hi) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    bf16x2 r = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-    return __builtin_bit_cast(uint32_t, r);
-  }
-  // acc + lo + hi of a packed pair (v_dot2c_f32_bf16 against (1, 1)).
-  static __device__ __forceinline__ float sum2(uint32_t p, float acc) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, p),
-                                           __builtin_bit_cast(bf16x2, 0x3f803f80u), acc, false);
-  }
-};
-template <> struct Mfma<f16_t> {
-  static __device__ __forceinline__ f32x16 run(u32x4 a, u32x4 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint32_t pack(float lo, float hi) {
-    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-    f16x2 r = {static_cast<_Float16>(lo), static_cast<_Float16>(hi)};
-    return __builtin_bit_cast(uint32_t, r);
-  }
-  // acc + lo + hi of a packed pair (v_dot2c_f32_f16 against (1, 1)).
-  static __device__ __forceinline__ float sum2(uint32_t p, float acc) {
-    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, p),
-                                  __builtin_bit_cast(f16x2, 0x3c003c00u), acc, false);
-  }
-};
-
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
 // LDS geometry, per stage: a K tile [64 keys][D] and a V tile [64 keys][D],
 // both row-major as they lie in memory.
 //  - K rows are padded by 8 elements (272 B for D=128): the QK^T A operand is
@@ -182,15 +144,6 @@ struct KvSrc {
   int c_ss2, k_sl2, v_sl2;  // row strides in bytes
   int n_ct;                 // cache tiles: ceil(cache_len / kBN)
 };
-
-constexpr int kBufWord3 = 0x00020000;  // gfx9-family raw buffer descriptor word 3
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const uint16_t* base, int rows,
-                                                           int row_bytes, int D) {
-  const int bytes = rows > 0 ? (rows - 1) * row_bytes + D * 2 : 0;
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), (short)0, bytes,
-                                           kBufWord3);
-}
 
 // K/V tile loads of the decode kernel: each cache row is read once per call,
 // so the loads are marked non-temporal (cache policy bit NT = 2).
@@ -469,32 +422,6 @@ struct PairDma {
   }
 };
 
-// Transposing LDS read (gfx950 ds_read_b64_tr_b16). Within each group of 16
-// lanes, lane i receives element i % 4 of the 8-byte chunks addressed by
-// lanes 4e + i / 4, e = 0..3 of its group.
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ u32x2 lds_read_tr16(const uint16_t* p) {
-  typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-  const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (lds_v4i16*)((__attribute__((address_space(3))) uint16_t*)(p)));
-  return __builtin_bit_cast(u32x2, r);
-}
-
-// LDS accesses by byte address (for the swizzled layout, whose addresses are
-// built with XOR).
-typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return uint32_t(uintptr_t((__attribute__((address_space(3))) const void*)(p)));
-}
-__device__ __forceinline__ u32x4 lds_read_b128_at(uint32_t addr) {
-  return *reinterpret_cast<const lds_u32x4*>(addr);
-}
-__device__ __forceinline__ u32x2 lds_read_tr16_at(uint32_t addr) {
-  typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-  const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_v4i16*>(addr));
-  return __builtin_bit_cast(u32x2, r);
-}
-
 // A row area in LDS: rows of D 16-bit elements, K-swizzled (chunk c of row r
 // at c ^ kswz(r), conflict-free for the K-operand read pattern and for 8-byte
 // writes of 32 rows). The kernels stage their result rows in one after the
@@ -675,26 +602,6 @@ __device__ __forceinline__ void qk_tile(const uint16_t* Ks, const u32x4 (&qr)[D 
     s[i / KS] = Mfma<T>::run(kf[i % W], qr[i % KS], s[i / KS]);
     if (i + W < N) kf[i % W] = frag(i + W);
   }
-}
-
-// Key of register r of half kt: row 32 kt + 8 (r / 4) + 4 g + r % 4 of the
-// tile, visible iff that row is below lim_rel (rows past the tile's valid
-// keys or past this query's visible end are not). ``lim`` is lim_rel - 4 g.
-__device__ __forceinline__ bool key_hidden(int kt, int r, int lim) {
-  return 32 * kt + 8 * (r / 4) + (r % 4) >= lim;
-}
-
-// Combine lanes i and i ^ 32 (v_permlane32_swap: a VALU exchange of the two
-// wave halves, with no trip through the LDS queue as ds_bpermute takes).
-__device__ __forceinline__ float xor32_max(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
-                                                  false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float xor32_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
-                                                  false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
 // Returns the exponent base (max in log2 units, 0 while nothing is visible).
@@ -4078,7 +3985,11 @@ int attention_entry(const void* q, int64_t q_sb, int64_t q_sl, int64_t q_sh, con
     a.cache_len_dev = cache_len_dev;
     a.n_seg = cache_lens ? int(B) : 0;
     for (int64_t i = 0; cache_lens && i < B; ++i) a.seg_cache[i] = int(cache_lens[i]);
-    const hipError_t e = launch_any(a, dtype, int(D), pa, static_cast<hipStream_t>(stream));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const bool wide = D == 256 && dtype != DX_F32 && tuning(DX_TUNE_ATTN_SPLITS) == 0 &&
+                      wide_fits(B, Lq, Lk, H, cache_len, cache_lens, n_blocks, causal != 0,
+                                device_cus());
+    const hipError_t e = wide ? launch_wide(a, dtype, st) : launch_any(a, dtype, int(D), pa, st);
     if (e != hipSuccess) {
       set_error("attention: launch failed: %s", hipGetErrorString(e));
       return DX_ELAUNCH;

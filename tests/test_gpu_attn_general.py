@@ -227,3 +227,57 @@ def test_general_kernel_leaves_the_counter_region_alone(device, built_lib):
     cb = _rand((2, 1, 2400, 8, 128), torch.bfloat16, 1.0, 98)
     gotb, refb = _run(device, qb, kb, vb, cb, 2400)
     _check(gotb, refb, torch.bfloat16, "bf16 after the general kernel")
+
+
+# The prefill kernel of head dim 256 (attn_wide.hip: 128 queries per work item, two
+# streams of 32-key tiles) at the edges of its tiles. Enough heads that the planner
+# takes it (a forced split count goes to the general kernel, the other side here).
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,lq,lk,h,hkv,cache_len,mask", [
+    (1, 1, 1, 64, 64, 0, None), (1, 33, 33, 64, 8, 0, "causal"), (1, 127, 127, 32, 32, 31, None),
+    (2, 129, 129, 24, 12, 40, [0, 50, 100]), (1, 257, 64, 24, 24, 0, None),
+    (1, 200, 200, 32, 32, 33, "causal"), (1, 96, 96, 64, 64, 20, [40, 0, 70]),
+    (1, 80, 80, 64, 64, 10, [-30, 20]), (1, 130, 130, 272, 16, 0, "causal"),
+])
+def test_wide_heads_prefill(device, built_lib, dtype, b, lq, lk, h, hkv, cache_len, mask):
+    g = torch.Generator().manual_seed(lq + h)
+    rand = lambda *s: torch.randn(s, generator=g).to(dtype)  # noqa: E731
+    q = rand(b, h, lq, 256).transpose(1, 2)  # head-major in memory
+    kv = rand(b, lk, 2, hkv, 256)            # k and v as slices of one projection
+    cache = rand(2, b, cache_len + 3, hkv, 256) if cache_len else None
+    bb = torch.tensor(mask) if isinstance(mask, list) else None
+    causal = mask == "causal"
+    ref = oatt.blockwise_causal_attention(q, kv[:, :, 0], kv[:, :, 1], cache, cache_len, bb, None,
+                                          causal, keep_fp32=True)
+    dev = lambda t: None if t is None else t.to(device)  # noqa: E731
+    qd, kvd = dev(q), dev(kv)
+    call = lambda: ops.blockwise_causal_attention(  # noqa: E731
+        qd, kvd[:, :, 0], kvd[:, :, 1], kv_cache=dev(cache), cache_len=cache_len,
+        block_boundaries=dev(bb), causal=causal)
+    got = call()
+    with _lib.tuning(_lib.TUNE_ATTN_SPLITS, 1):
+        general = call()
+    seen = ~torch.isnan(ref)
+    assert torch.equal(torch.isnan(got.cpu()), ~seen)
+    assert torch.equal(torch.isnan(general.cpu()), ~seen)
+    assert not torch.equal(got.cpu()[seen], general.cpu()[seen]) or lq * lk == 1
+    for what, other in (("oracle", ref), ("general kernel", general.float().cpu())):
+        assert_parity(got.cpu()[seen], other[seen], what=f"{what} {lq}x{lk}+{cache_len} {mask}")
+
+
+@pytest.mark.parametrize("scale", [-0.05, 0.0])
+def test_wide_heads_scales_cursor_ragged(device, built_lib, scale):
+    q, k, v = (torch.randn(2, 140, 32, 256, device=device).bfloat16() for _ in range(3))
+    cache = torch.randn(2, 2, 100, 32, 256, device=device).bfloat16()
+    kw = dict(softmax_scale=scale, block_boundaries=torch.tensor([0, 83], device=device))
+    host = ops.blockwise_causal_attention(q, k, v, kv_cache=cache, cache_len=70, **kw)
+    cursor = torch.tensor([70], dtype=torch.int32, device=device)
+    assert torch.equal(host, ops.blockwise_causal_attention(q, k, v, kv_cache=cache,
+                                                            cache_len=cursor, **kw))
+    rag = ops.blockwise_causal_attention_varlen(q, k, v, kv_cache=cache, cache_lens=[70, 9], **kw)
+    assert torch.equal(rag[:1], host[:1])
+    for i, c in enumerate((70, 9)):
+        ref = oatt.blockwise_causal_attention(
+            q[i:i + 1].cpu(), k[i:i + 1].cpu(), v[i:i + 1].cpu(), cache[:, i:i + 1].cpu(), c,
+            kw["block_boundaries"].cpu(), scale, False, keep_fp32=True)
+        assert_parity(rag[i:i + 1], ref, what=f"seq {i}")
