@@ -3986,10 +3986,18 @@ int attention_entry(const void* q, int64_t q_sb, int64_t q_sl, int64_t q_sh, con
     a.n_seg = cache_lens ? int(B) : 0;
     for (int64_t i = 0; cache_lens && i < B; ++i) a.seg_cache[i] = int(cache_lens[i]);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const bool wide = D == 256 && dtype != DX_F32 && tuning(DX_TUNE_ATTN_SPLITS) == 0 &&
+    // The kernels of attn_f32.hip and attn_wide.hip where they are the faster
+    // ones; a forced split count keeps the general kernel.
+    const bool free_form = tuning(DX_TUNE_ATTN_SPLITS) == 0;
+    F32Plan pf{};
+    if (dtype == DX_F32 && free_form)
+      pf = plan_f32(B, Lq, Lk, H, D, cache_len, cache_lens, n_blocks, causal != 0, device_cus());
+    const bool wide = D == 256 && dtype != DX_F32 && free_form &&
                       wide_fits(B, Lq, Lk, H, cache_len, cache_lens, n_blocks, causal != 0,
                                 device_cus());
-    const hipError_t e = wide ? launch_wide(a, dtype, st) : launch_any(a, dtype, int(D), pa, st);
+    const hipError_t e = pf.fits ? launch_f32(a, int(D), pf, st)
+                         : wide  ? launch_wide(a, dtype, st)
+                                 : launch_any(a, dtype, int(D), pa, st);
     if (e != hipSuccess) {
       set_error("attention: launch failed: %s", hipGetErrorString(e));
       return DX_ELAUNCH;

@@ -281,3 +281,48 @@ def test_wide_heads_scales_cursor_ragged(device, built_lib, scale):
             q[i:i + 1].cpu(), k[i:i + 1].cpu(), v[i:i + 1].cpu(), cache[:, i:i + 1].cpu(), c,
             kw["block_boundaries"].cpu(), scale, False, keep_fp32=True)
         assert_parity(rag[i:i + 1], ref, what=f"seq {i}")
+
+
+# The fp32 kernel that deals 16-key tiles to a workgroup's waves (attn_f32.hip) at the
+# edges of its tiles and in each of its forms (eight waves; four waves past one item per
+# CU; two query tiles per item past 700 items; head dim 256). Bar: fp32 sums in another
+# order, a few 1e-7 of values of size one, as the general kernel's tests.
+@pytest.mark.parametrize("d", [32, 64, 128, 256])
+@pytest.mark.parametrize("b,lq,lk,h,hkv,cache_len,mask", [
+    (1, 1, 1, 8, 8, 0, None), (1, 17, 17, 24, 3, 15, "causal"), (2, 33, 33, 12, 12, 17, [0, 16, 32]),
+    (1, 83, 130, 12, 4, 0, None), (1, 96, 96, 8, 8, 20, [40, 0, 70]), (1, 80, 80, 8, 8, 10, [-30, 20]),
+    (1, 100, 100, 48, 48, 40, "causal"), (1, 97, 97, 104, 8, 3, [0, 50]),
+])
+def test_fp32_wave_split(device, built_lib, d, b, lq, lk, h, hkv, cache_len, mask):
+    g = torch.Generator().manual_seed(lq + h + d)
+    rand = lambda *s: torch.randn(s, generator=g)  # noqa: E731
+    q = rand(b, h, lq, d).transpose(1, 2)  # head-major in memory
+    kv = rand(b, lk, 2, hkv, d)            # k and v as slices of one projection
+    cache = rand(2, b, cache_len + 3, hkv, d) if cache_len else None
+    bb = torch.tensor(mask) if isinstance(mask, list) else None
+    causal = mask == "causal"
+    ref = oatt.blockwise_causal_attention(q, kv[:, :, 0], kv[:, :, 1], cache, cache_len, bb, None,
+                                          causal, keep_fp32=True)
+    dev = lambda t: None if t is None else t.to(device)  # noqa: E731
+    qd, kvd = dev(q), dev(kv)
+    call = lambda: ops.blockwise_causal_attention(  # noqa: E731
+        qd, kvd[:, :, 0], kvd[:, :, 1], kv_cache=dev(cache), cache_len=cache_len,
+        block_boundaries=dev(bb), causal=causal)
+    got = call()
+    with _lib.tuning(_lib.TUNE_ATTN_SPLITS, 1):
+        general = call()
+    seen = ~torch.isnan(ref)
+    assert torch.equal(torch.isnan(got.cpu()), ~seen)
+    for what, other in (("oracle", ref), ("general kernel", general.cpu())):
+        assert_parity(got.cpu()[seen], other[seen], max_abs=1e-5, mean_abs=1e-6,
+                      what=f"{what} D={d} {lq}x{lk}+{cache_len} {mask}")
+
+
+def test_fp32_wave_split_masks_nonfinite_future_keys(device, built_lib):
+    q, k, v = (torch.randn(1, 64, 8, 64, device=device) for _ in range(3))
+    bb = torch.tensor([0, 32], device=device)
+    base = ops.blockwise_causal_attention(q, k, v, block_boundaries=bb)
+    k2, v2 = k.clone(), v.clone()
+    k2[:, 32:], v2[:, 32:] = float("inf"), float("nan")
+    got = ops.blockwise_causal_attention(q, k2, v2, block_boundaries=bb)
+    assert torch.equal(got[:, :32], base[:, :32])
