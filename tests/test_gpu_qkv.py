@@ -241,6 +241,9 @@ def test_self_attention_fused_projection_matches_unfused(device, built_lib, writ
     (2, 32, 1536, 1536, DT, True), (1, 65, 1024, 128, DT, True), (1, 83, 3072, 3072, DT, True),
     (4, 24, 2560, 2576, DT, False), (1, 128, 4096, 4096, torch.float16, True),
     (1, 113, 512, 8208, DT, True),  # token tiles and feature tiles both end mid-group
+    # waves with one, two and three staged pieces in one workgroup
+    (1, 43, 3072, 3072, torch.float16, True), (1, 72, 3072, 3072, DT, True),
+    (1, 70, 2048, 8192, DT, False),
 ])
 def test_linear_chunk(device, built_lib, b, l, c, n, dtype, bias):
     """``F.linear`` of a chunk, one rounding of the exact sum: within one ulp of the 64-bit
