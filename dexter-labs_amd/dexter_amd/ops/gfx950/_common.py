@@ -21,11 +21,14 @@ MATRIX_DTYPES = (torch.bfloat16, torch.float16)
 
 def rows_ok(t: torch.Tensor) -> bool:
     """Last dim contiguous and every other stride keeps 16-byte row alignment."""
-    if t.stride(-1) != 1 and t.shape[-1] != 1:
+    steps, sizes = t.stride(), t.shape
+    if (steps[-1] != 1 and sizes[-1] != 1) or t.data_ptr() % 16:
         return False
     per16 = 16 // t.element_size()
-    return (t.data_ptr() % 16 == 0
-            and all(s % per16 == 0 for s, n in zip(t.stride()[:-1], t.shape[:-1]) if n > 1))
+    for i in range(len(steps) - 1):
+        if steps[i] % per16 and sizes[i] > 1:
+            return False
+    return True
 
 
 def as_rows(t: torch.Tensor) -> torch.Tensor:
@@ -35,7 +38,21 @@ def as_rows(t: torch.Tensor) -> torch.Tensor:
 
 def strides(t: torch.Tensor, dims: int) -> list[int]:
     """The first ``dims`` strides; a size-1 dim gets stride 0 (it is never stepped)."""
-    return [0 if t.shape[i] == 1 else t.stride(i) for i in range(dims)]
+    steps, sizes = t.stride(), t.shape
+    return [0 if sizes[i] == 1 else steps[i] for i in range(dims)]
+
+
+def flat_as(t: torch.Tensor, device: torch.device, dtype: torch.dtype) -> torch.Tensor:
+    """``t`` as one contiguous row of ``dtype`` on ``device``: itself when it is that
+    already (each conversion that changes nothing still costs about a microsecond)."""
+    if t.dim() == 1 and t.dtype == dtype and t.device == device and t.is_contiguous():
+        return t
+    return t.reshape(-1).to(device=device, dtype=dtype).contiguous()
+
+
+def moved(t: torch.Tensor, device: torch.device, dtype: torch.dtype) -> torch.Tensor:
+    """``t.to(device, dtype)``, without the call when nothing changes."""
+    return t if t.dtype == dtype and t.device == device else t.to(device=device, dtype=dtype)
 
 
 def device_cursor(t: torch.Tensor, device: torch.device, what: str) -> torch.Tensor:

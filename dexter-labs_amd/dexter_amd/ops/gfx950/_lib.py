@@ -226,7 +226,11 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream of ``device`` as an address, read anew on every call (the raw
+    getter: building a ``torch.cuda.Stream`` only to take its address costs 2 us)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if index is None else index)
 
 
 _tuning_values: dict[int, int] = {}

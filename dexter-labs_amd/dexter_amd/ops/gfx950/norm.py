@@ -35,15 +35,30 @@ _MAX_BATCH_GRID = 65535
 
 
 def _max_cols(dtype: torch.dtype) -> int:
-    per_pack = 16 // torch.empty((), dtype=dtype).element_size()
+    per_pack = 16 // dtype.itemsize
     return _PACKS_PER_LANE * 64 * per_pack * _MAX_WAVES
 
 
 def _promote(*dtypes: torch.dtype) -> torch.dtype:
     out = dtypes[0]
     for d in dtypes[1:]:
-        out = torch.promote_types(out, d)
+        if d is not out:
+            out = torch.promote_types(out, d)
     return out
+
+
+def _broadcast(*shapes: torch.Size) -> torch.Size:
+    """``torch.broadcast_shapes``, with its error for shapes that do not fit. Its checks cost
+    10 us for three shapes, and each op needs it twice; these loops cost 2."""
+    out = list(max(shapes, key=len))
+    for shape in shapes:
+        off = len(out) - len(shape)
+        for i, n in enumerate(shape):
+            if n != 1 and n != out[off + i]:
+                if out[off + i] != 1:
+                    return torch.broadcast_shapes(*shapes)
+                out[off + i] = n
+    return torch.Size(out)
 
 
 def _broadcast_ok(x, *others) -> bool:
@@ -54,7 +69,7 @@ def _broadcast_ok(x, *others) -> bool:
     if x.dim() == 0:
         return False
     try:
-        shape = torch.broadcast_shapes(*(t.shape for t in tensors))
+        shape = _broadcast(*(t.shape for t in tensors))
     except RuntimeError:
         return False
     cols = x.shape[-1]
@@ -74,6 +89,14 @@ def _rows3(t: torch.Tensor, shape: torch.Size, b: int, seq: int) -> tuple[torch.
     batch and row strides in elements. Broadcast dims keep stride 0 (no copy); a copy is
     made only when the last dim is not contiguous or the leading dims cannot be merged."""
     cols = shape[-1]
+    if len(shape) == 3 and shape[0] == b:
+        # [b, seq, C] already: the strides of the expanded view, without making it.
+        sizes, steps = t.shape, t.stride()
+        n = len(sizes)
+        if n > 0 and sizes[-1] == cols and (cols == 1 or steps[-1] == 1):
+            sb = steps[-3] if n == 3 and sizes[0] != 1 else 0
+            sl = steps[-2] if n > 1 and sizes[-2] != 1 else 0
+            return t, sb, sl
     e = t.expand(shape).reshape(b, seq, cols)
     if cols > 1 and e.stride(-1) != 1:
         e = e.contiguous()
@@ -98,12 +121,13 @@ def _row_grid(shape: torch.Size) -> tuple[int, int]:
 @register("norm", "adaln", name="hip_adaln_gfx950",
           capability=CDNA4, priority=Priority.SPECIALISED, accepts=_accepts_adaln)
 def adaln_modulate(x, scale, shift, eps):
-    shape = torch.broadcast_shapes(x.shape, scale.shape, shift.shape)
+    shape = _broadcast(x.shape, scale.shape, shift.shape)
     if shape[-1] != x.shape[-1]:
         raise ValueError(f"scale/shift {tuple(scale.shape)}/{tuple(shift.shape)} must broadcast "
                          f"to rows of x {tuple(x.shape)}")
     mdt = _promote(scale.dtype, shift.dtype)
-    scale, shift = scale.to(mdt), shift.to(mdt)
+    scale = scale if scale.dtype is mdt else scale.to(mdt)
+    shift = shift if shift.dtype is mdt else shift.to(mdt)
     odt = _promote(x.dtype, mdt)
     b, seq = _row_grid(shape)
     cols = shape[-1]
@@ -113,12 +137,11 @@ def adaln_modulate(x, scale, shift, eps):
     xv, x_sb, x_sl = _rows3(x, shape, b, seq)
     sc, sc_sb, sc_sl = _rows3(scale, shape, b, seq)
     sh, sh_sb, sh_sl = _rows3(shift, shape, b, seq)
-    o3 = out.view(b, seq, cols)
     lib = _lib.load()
     rc = lib.dx_adaln_modulate(
         xv.data_ptr(), x_sb, x_sl, _lib.dtype_code(x.dtype),
         sc.data_ptr(), sc_sb, sc_sl, sh.data_ptr(), sh_sb, sh_sl, _lib.dtype_code(mdt),
-        o3.data_ptr(), o3.stride(0), o3.stride(1), _lib.dtype_code(odt),
+        out.data_ptr(), seq * cols, cols, _lib.dtype_code(odt),
         b, seq, cols, float(eps), _lib.stream_handle(x.device))
     _lib.check(rc, "adaln_modulate")
     return out
@@ -127,12 +150,13 @@ def adaln_modulate(x, scale, shift, eps):
 @register("norm", "gated_residual", name="hip_gated_residual_gfx950",
           capability=CDNA4, priority=Priority.SPECIALISED, accepts=_accepts_gated)
 def gated_residual(x, y, gate):
-    shape = torch.broadcast_shapes(x.shape, y.shape, gate.shape)
+    shape = _broadcast(x.shape, y.shape, gate.shape)
     if shape[-1] != x.shape[-1]:
         raise ValueError(f"y/gate {tuple(y.shape)}/{tuple(gate.shape)} must broadcast to rows "
                          f"of x {tuple(x.shape)}")
     xdt = _promote(x.dtype, y.dtype)
-    x, y = x.to(xdt), y.to(xdt)
+    x = x if x.dtype is xdt else x.to(xdt)
+    y = y if y.dtype is xdt else y.to(xdt)
     odt = _promote(xdt, gate.dtype)
     b, seq = _row_grid(shape)
     cols = shape[-1]
@@ -142,12 +166,11 @@ def gated_residual(x, y, gate):
     xv, x_sb, x_sl = _rows3(x, shape, b, seq)
     yv, y_sb, y_sl = _rows3(y, shape, b, seq)
     gv, g_sb, g_sl = _rows3(gate, shape, b, seq)
-    o3 = out.view(b, seq, cols)
     lib = _lib.load()
     rc = lib.dx_gated_residual(
         xv.data_ptr(), x_sb, x_sl, yv.data_ptr(), y_sb, y_sl, _lib.dtype_code(xdt),
         gv.data_ptr(), g_sb, g_sl, _lib.dtype_code(gate.dtype),
-        o3.data_ptr(), o3.stride(0), o3.stride(1), _lib.dtype_code(odt),
+        out.data_ptr(), seq * cols, cols, _lib.dtype_code(odt),
         b, seq, cols, _lib.stream_handle(x.device))
     _lib.check(rc, "gated_residual")
     return out

@@ -26,15 +26,18 @@ import torch
 
 from ...registry import Priority, register
 from . import _lib
-from ._common import CDNA4, MATRIX_DTYPES, device_cursor, rows_ok, strides
+from ._common import CDNA4, MATRIX_DTYPES, device_cursor, flat_as, moved, rows_ok, strides
 
 _TABLE_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 MAX_TOKENS = 128
 
 
 def _weight_ok(w, hd, c, dtype) -> bool:
-    return (w.dim() == 2 and tuple(w.shape) == (hd, c) and w.dtype == dtype and w.is_cuda
-            and w.stride(1) == 1 and w.data_ptr() % 16 == 0 and w.stride(0) % 8 == 0)
+    if w.dim() != 2:
+        return False
+    rows, step = w.stride()
+    return (w.shape == (hd, c) and w.dtype == dtype and w.is_cuda
+            and step == 1 and w.data_ptr() % 16 == 0 and rows % 8 == 0)
 
 
 def _accepts(x, wq, bq, wk, bk, wv, bv, q_weight, k_weight, cos, sin, heads, *args,
@@ -54,7 +57,7 @@ def _bias(t, hd, dtype, device):
         return None
     if t.numel() != hd:
         raise ValueError(f"bias must have {hd} elements, got {t.numel()}")
-    return t.reshape(-1).to(device=device, dtype=dtype).contiguous()
+    return flat_as(t, device, dtype)
 
 
 @register("rope", "qkv_norm_rope", name="hip_qkv_norm_rope_gfx950",
@@ -67,8 +70,8 @@ def qkv_norm_rope(x, wq, bq, wk, bk, wv, bv, q_weight, k_weight, cos, sin, heads
     if not rows_ok(x):
         x = x.contiguous()
     wdt = q_weight.dtype if q_weight.dtype in _TABLE_DTYPES else torch.float32
-    qw = q_weight.reshape(-1).to(device=x.device, dtype=wdt).contiguous()
-    kw = k_weight.reshape(-1).to(device=x.device, dtype=wdt).contiguous()
+    device = x.device
+    qw, kw = flat_as(q_weight, device, wdt), flat_as(k_weight, device, wdt)
     if qw.numel() != hd or kw.numel() != hd:
         raise ValueError(f"norm weights must have H*D = {hd} elements")
     tdt = cos.dtype if cos.dtype in _TABLE_DTYPES else torch.float32
@@ -76,10 +79,10 @@ def qkv_norm_rope(x, wq, bq, wk, bk, wv, bv, q_weight, k_weight, cos, sin, heads
     for t in (cos, sin):
         if t.dim() != 2 or t.shape[-1] != dim // 2 or t.shape[0] not in (seq, 1):
             raise ValueError(f"cos/sin must be [L, D/2] = [{seq}, {dim // 2}], got {tuple(t.shape)}")
-        t = t.to(device=x.device, dtype=tdt)
+        t = moved(t, device, tdt)
         tables.append(t if rows_ok(t) else t.contiguous())
     cs, sn = tables
-    biases = [_bias(t, hd, x.dtype, x.device) for t in (bq, bk, bv)]
+    biases = [_bias(t, hd, x.dtype, device) for t in (bq, bk, bv)]
     q_out = torch.empty((b, seq, heads, dim), device=x.device, dtype=x.dtype)
     k_out = torch.empty_like(q_out)
     v_out = torch.empty_like(q_out)

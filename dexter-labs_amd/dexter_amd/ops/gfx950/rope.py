@@ -23,16 +23,17 @@ import torch
 
 from ...registry import Priority, register
 from . import _lib
-from ._common import CDNA4, MATRIX_DTYPES, as_rows, device_cursor, strides
+from ._common import CDNA4, MATRIX_DTYPES, as_rows, device_cursor, flat_as, moved, strides
 
 _TABLE_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 _MAX_PLANE = 256 * 4 * 16
 
 
 def _accepts(q, k, *args, **kwargs) -> bool:
+    shape = q.shape
     return (q.is_cuda and k.is_cuda and q.dtype in MATRIX_DTYPES and k.dtype == q.dtype
-            and q.dim() == 4 and q.shape == k.shape and q.shape[-1] % 16 == 0
-            and q.shape[2] * q.shape[3] <= _MAX_PLANE)
+            and len(shape) == 4 and shape == k.shape and shape[3] % 16 == 0
+            and shape[2] * shape[3] <= _MAX_PLANE)
 
 
 def _accepts_append(q, k, v, cache, *args, **kwargs) -> bool:
@@ -47,14 +48,14 @@ def _prepare(q, k, q_weight, k_weight, cos, sin):
     if q_weight.numel() != heads * dim or k_weight.numel() != heads * dim:
         raise ValueError(f"norm weights must have H*D = {heads * dim} elements")
     wdt = q_weight.dtype if q_weight.dtype in _TABLE_DTYPES else torch.float32
-    qw = q_weight.reshape(-1).to(device=q.device, dtype=wdt).contiguous()
-    kw = k_weight.reshape(-1).to(device=q.device, dtype=wdt).contiguous()
+    device = q.device
+    qw, kw = flat_as(q_weight, device, wdt), flat_as(k_weight, device, wdt)
     tdt = cos.dtype if cos.dtype in _TABLE_DTYPES else torch.float32
     tables = []
     for t in (cos, sin):
         if t.dim() != 2 or t.shape[-1] != dim // 2 or t.shape[0] not in (seq, 1):
             raise ValueError(f"cos/sin must be [L, D/2] = [{seq}, {dim // 2}], got {tuple(t.shape)}")
-        tables.append(as_rows(t.to(device=q.device, dtype=tdt)))
+        tables.append(as_rows(moved(t, device, tdt)))
     return as_rows(q), as_rows(k), qw, kw, tables[0], tables[1], tdt
 
 

@@ -147,9 +147,11 @@ class Capability:
     def satisfied_by(self, platform: PlatformInfo) -> bool:
         if self.vendors is not None and platform.vendor not in self.vendors:
             return False
-        if self.min_arch is not None and platform.arch_version < self.min_arch:
+        arch = (platform.arch_version.major, platform.arch_version.minor)
+        low, high = self.min_arch, self.max_arch
+        if low is not None and arch < (low.major, low.minor):
             return False
-        if self.max_arch is not None and platform.arch_version > self.max_arch:
+        if high is not None and arch > (high.major, high.minor):
             return False
         return self.features <= platform.features
 

@@ -202,9 +202,11 @@ def select_spec(family: str, mode: str, *args, **kwargs) -> KernelSpec:
             if spec.name == pin:
                 return spec
         raise LookupError(f"{PIN_ENV} pinned {key}:{pin}, which is not available here")
-    for ruling in _rulings(key, platform, args, kwargs):
-        if ruling.status == ELIGIBLE:
-            return ruling.spec
+    # The pass of _rulings without its report: the first spec it would call eligible.
+    for spec in _CATALOGUE.specs(key):
+        if spec.capability.satisfied_by(platform) and (
+                spec.accepts is None or spec.accepts(*args, **kwargs)):
+            return spec
     names = [s.name for s in _CATALOGUE.specs(key)]
     raise LookupError(f"no kernel for {key} on {platform.describe()}. "
                       f"Registered: {names or 'none'}")
