@@ -22,10 +22,20 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.autograd import forward_ad
 
 from .. import ops
 from ..registry import select
 from .kv_cache import KVCache
+
+
+def _computes_only(*params) -> bool:
+    """Whether a torch op on ``params`` would do no more than compute (``forward`` runs
+    without gradients): no autocast, no forward-mode level, no functorch transform and no
+    tensor subclass, all of which a kernel called by address passes by."""
+    return (not torch.is_autocast_enabled("cuda") and forward_ad._current_level < 0
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and all(p is None or type(p) in (nn.Parameter, torch.Tensor) for p in params))
 
 
 class SelfAttention(nn.Module):
@@ -103,7 +113,8 @@ class SelfAttention(nn.Module):
         x = out.flatten(2)
         b, seq, dim = x.shape
         linear = F.linear
-        if 0 < b * seq <= 128 and dim % 512 == 0 and dim <= 4096:
+        if 0 < b * seq <= 128 and dim % 512 == 0 and dim <= 4096 \
+                and _computes_only(self.o.weight, self.o.bias):
             try:
                 linear = select("gemm", "linear_chunk", x, self.o.weight, self.o.bias)
             except LookupError:  # a weight layout the kernel does not take

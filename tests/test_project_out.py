@@ -1,0 +1,64 @@
+"""Which output projections go to the chunk kernel (the choice alone, no GPU)."""
+
+import contextlib
+
+import pytest
+import torch
+import torch.nn.functional as F
+from torch.autograd import forward_ad
+
+from dexter_amd.models import attention
+
+
+def _project(monkeypatch, tokens, dim, edit=lambda m: None):
+    module = attention.SelfAttention(dim, dim // 64, dtype=torch.float32)
+    edit(module)
+    calls = []
+
+    def select(family, mode, *args):
+        calls.append((family, mode))
+        return F.linear
+
+    monkeypatch.setattr(attention, "select", select)
+    with torch.no_grad():
+        out = module._project_out(torch.randn(1, tokens, dim // 64, 64))
+    assert out.shape == (1, tokens, dim)
+    return calls
+
+
+@pytest.mark.parametrize("tokens,dim,chunk", [
+    (1, 512, True), (128, 512, True), (129, 512, False), (0, 512, False), (8, 576, False)])
+def test_sizes(monkeypatch, tokens, dim, chunk):
+    assert _project(monkeypatch, tokens, dim) == ([("gemm", "linear_chunk")] if chunk else [])
+
+
+@pytest.mark.parametrize("inside", ["autocast", "forward_ad", "vmap"])
+def test_torch_transforms_keep_torchs_linear(monkeypatch, inside):
+    if inside == "vmap":
+        calls = []
+
+        def one(x):
+            calls.append(_project(monkeypatch, 8, 512))
+            return x
+
+        torch.vmap(one, randomness="same")(torch.zeros(2))
+        assert calls == [[]]
+        return
+    with contextlib.ExitStack() as stack:
+        stack.enter_context(torch.autocast("cuda", dtype=torch.bfloat16)
+                            if inside == "autocast" else forward_ad.dual_level())
+        if inside == "autocast" and not torch.is_autocast_enabled("cuda"):
+            pytest.skip("torch turns CUDA autocast off without a device")
+        assert _project(monkeypatch, 8, 512) == []
+
+
+def test_a_weight_subclass_keeps_torchs_linear(monkeypatch):
+    class Tagged(torch.Tensor):
+        pass
+
+    def edit(m):
+        w = m.o.weight.data.as_subclass(Tagged)
+        del m.o.weight
+        m.o.weight = w
+
+    assert _project(monkeypatch, 8, 512, edit) == []
