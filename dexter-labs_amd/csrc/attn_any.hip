@@ -1,7 +1,11 @@
 // The general attention kernels for gfx950: the calls that the 16-bit MFMA
 // kernels (attn_fwd.hip) do not take -- fp32 inputs at any supported head
 // dim, and bf16/f16 inputs at head dims 16, 32 and 256 -- under the same
-// arguments and the same mask rules (attn_common.h). attn_any_kernel works in
+// arguments and the same mask rules (attn_common.h). Two classes of them have
+// kernels of their own where the sizes favour those (plan_f32, wide_fits): fp32
+// at head dims 32 to 256 (attn_f32.hip) and 16-bit prefill at head dim 256
+// (attn_wide.hip); the rest, and every forced split count, run here.
+// attn_any_kernel works in
 // fp32 from end to end (fp32 inputs, and 16-bit inputs at head dim 16);
 // attn_any16_kernel multiplies 16-bit inputs at head dims 32 and 256 on the
 // 16-bit MFMA with fp32 sums (described at its definition). The reference op is dtype-generic (ops/reference/attention.py:

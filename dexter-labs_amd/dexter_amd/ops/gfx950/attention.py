@@ -34,7 +34,8 @@ Two cases the reference op cannot take are defined as its callers use them:
 
 Inputs in bf16 or f16 at head dim 64 or 128 run on the bf16/f16 MFMA kernels;
 fp32 inputs (any supported head dim) and bf16/f16 at head dims 16, 32 and 256
-run on the general kernel (fp32 MFMA, fp32 softmax; ``csrc/attn_any.hip``), as
+run on the general kernels (``csrc/attn_any.hip``, ``attn_f32.hip``,
+``attn_wide.hip``: fp32 softmax and sums), as
 the reference op is dtype-generic (``ops/reference/attention.py:62-77``) and
 the Triton kernel takes any power-of-two head dim
 (``blockwise_causal.py:162-172``).

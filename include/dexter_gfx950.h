@@ -207,7 +207,8 @@ int dx_kv_append(const void* k, int64_t k_sb, int64_t k_sl, int64_t k_sh,
  * at D 64 or 128 run on the 16-bit MFMA kernels; fp32 (any D) and bf16/f16 at
  * D 16, 32 or 256 on the general kernels (fp32 softmax and sums, products of
  * the inputs as they are: fp32, or 16-bit MFMA for bf16/f16 at D 32 and 256;
- * one rounding to dtype). Strides are multiples of 16 bytes.
+ * one rounding to dtype). Several kernels share each class of calls, chosen by
+ * the sizes; the choice changes no argument and no workspace. Strides are multiples of 16 bytes.
  * out may be strided like q. cache may be NULL when cache_len == 0.
  * workspace must hold dx_attention_workspace_bytes(...) bytes for the same
  * shape (it may be NULL when that is 0). Its first 256 KiB hold the
@@ -354,7 +355,7 @@ int dx_qk_norm_rope_append_dev(const void* q, int64_t q_sb, int64_t q_sl, int64_
  * the same cache_lens array (cache_len ignored) for the varlen entry point.
  * It takes no dtype: the bytes cover every dtype of the shape (at D 64 and
  * 128 an fp32 call splits its keys no further than fits the bf16/f16 plan's
- * bytes). The general kernel never writes the first 256 KiB (the counters).
+ * bytes). The general kernels never write the first 256 KiB (the counters).
  * Returns a negative DX_E* code on a bad shape.
  */
 int64_t dx_attention_workspace_bytes(int64_t B, int64_t Lq, int64_t Lk, int64_t H,
