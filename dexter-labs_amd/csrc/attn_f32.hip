@@ -314,7 +314,7 @@ hipError_t launch_d(const AttnArgs& a, const F32Plan& p, hipStream_t st) {
 // over 1083 40.5 -> 34.5, over 4083 95 -> 96 (stays); 664 x 24 heads 116 -> 61,
 // causal 75 -> 48; 2500 x 12 heads 414 -> 358. D 16 is not measured and stays.
 F32Plan plan_f32(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_t cache_len,
-                 const int64_t* cache_lens, int64_t n_blocks, bool causal, int cus) {
+                 const int64_t* cache_lens, int64_t n_blocks, bool causal, int cus, int form) {
   F32Plan p{};
   if (D < 32) return p;
   const int64_t items = B * H * ((Lq + 15) / 16);
@@ -322,8 +322,12 @@ F32Plan plan_f32(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_
   const bool many = D < 256 && items > 700;
   p.waves = D < 256 && items <= cus ? 8 : 4;
   p.qt = many ? 2 : 1;
-  p.fits = many;
-  if (many) return p;
+  if (form) {
+    p.waves = D < 256 && form == 8 ? 8 : 4;
+    p.qt = D < 256 && form == 2 ? 2 : 1;
+  }
+  p.fits = many || form;
+  if (p.fits) return p;
   auto tiles = [](int64_t keys) { return double((keys + kKeys - 1) / kKeys); };
   double seen = tiles(Lk);  // mean new-key tiles of an item
   if (causal) seen = (seen + 1) / 2;

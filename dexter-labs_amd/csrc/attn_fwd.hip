@@ -3361,8 +3361,18 @@ int device_cus() {
   return cache[dev];
 }
 
-// Attention kernels a plan can pick (the DX_TUNE_ATTN_KERNEL values).
-enum AttnKernel { kSingle = 1, kDual = 2, kPaired = 3, kDecode = 4, kWave = 5 };
+// Attention kernels a plan can pick (the DX_TUNE_ATTN_KERNEL values, and what
+// dx_attention_kernel reports): those of this file, then the general ones.
+enum AttnKernel {
+  kSingle = 1, kDual = 2, kPaired = 3, kDecode = 4, kWave = 5,
+  kGeneral = 6, kWide = 7, kF32Eight = 8, kF32Four = 9, kF32Pair = 10
+};
+
+// The forced kernel of this file's calls, or of the general ones; 0: none.
+int forced_kernel_of(bool general) {
+  const int f = tuning(DX_TUNE_ATTN_KERNEL);
+  return (f >= kGeneral) == general ? f : 0;
+}
 
 struct Plan {
   int n_qtiles;
@@ -3482,7 +3492,7 @@ Plan make_plan(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_t 
                const int64_t* cache_lens) {
   Plan p{};
   const int cus = device_cus();
-  const int forced_kernel = tuning(DX_TUNE_ATTN_KERNEL);
+  const int forced_kernel = forced_kernel_of(false);
   const int forced_splits = tuning(DX_TUNE_ATTN_SPLITS);
   // Segments: one per sequence of a ragged batch, longest first; a uniform
   // call is one segment of all B*H (batch, head) pairs.
@@ -3685,7 +3695,7 @@ bool wave_kernel_fits(double items, double tiles, int64_t D, int64_t nb, bool ca
 // workspace query knows no mask); this kernel leaves it untouched.
 void use_wave_kernel(Plan& p, int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D,
                      int64_t cache_len, int64_t n_blocks, bool causal) {
-  const int forced = tuning(DX_TUNE_ATTN_KERNEL);
+  const int forced = forced_kernel_of(false);
   if (forced ? forced != kWave
              : tuning(DX_TUNE_ATTN_SPLITS) != 0 || tuning(DX_TUNE_ATTN_PMERGE) != 0)
     return;
@@ -3720,6 +3730,68 @@ void use_wave_kernel(Plan& p, int64_t B, int64_t Lq, int64_t Lk, int64_t H, int6
   }
   p.partials = p.comb_blocks = p.counter_bytes = p.ws_bytes = 0;
   p.pmerge = p.spread = false;
+}
+
+// fp32 inputs and the other head dims take the general kernels.
+bool general_call(int dtype, int64_t D) { return dtype == DX_F32 || (D != 64 && D != 128); }
+
+// What decides a call's kernel: its shape, the form of its mask and q's row
+// stride (elements).
+struct CallShape {
+  int dtype;
+  int64_t B, Lq, Lk, H, D, cache_len;
+  const int64_t* cache_lens;
+  int64_t n_blocks;
+  bool causal;
+  int64_t q_sl;
+};
+
+struct Route {
+  int kernel = 0;        // AttnKernel
+  Plan p{};              // a kernel of this file
+  AnyPlan pa{};          // a general one
+  F32Plan pf{};          // attn_f32.hip's
+  int64_t ws_bytes = 0;  // workspace the call has to bring, whichever kernel takes it
+};
+
+// The kernel that a call with at least one query takes, and its plan.
+int route_call(const CallShape& c, Route& r) {
+  const int cus = device_cus();
+  if (!general_call(c.dtype, c.D)) {
+    r.p = make_plan(c.B, c.Lq, c.Lk, c.H, c.D, c.cache_len, c.cache_lens);
+    DX_CHECK_ARG(r.p.items < (int64_t(1) << 31), "attention: grid too large");
+    r.ws_bytes = r.p.ws_bytes;
+    use_wave_kernel(r.p, c.B, c.Lq, c.Lk, c.H, c.D, c.cache_len, c.n_blocks, c.causal);
+    r.kernel = r.p.kernel;
+    return DX_OK;
+  }
+  int64_t max_cache = c.cache_len;
+  if (c.cache_lens) max_cache = *std::max_element(c.cache_lens, c.cache_lens + c.B);
+  // The workspace query takes no dtype: at head dims 64 and 128 it reports
+  // the 16-bit kernels' bytes, and fp32 calls split no more than fits them.
+  const int64_t cap = c.D == 64 || c.D == 128
+                          ? make_plan(c.B, c.Lq, c.Lk, c.H, c.D, c.cache_len, c.cache_lens).ws_bytes
+                          : -1;
+  r.pa = plan_any(c.B, c.Lq, c.Lk, c.H, c.D, max_cache, cap, cus);
+  DX_CHECK_ARG(r.pa.items < (int64_t(1) << 31), "attention: grid too large");
+  r.ws_bytes = r.pa.ws_bytes;
+  // The kernels of attn_f32.hip and attn_wide.hip where they are the faster
+  // ones, or forced; a forced split count keeps the general kernel.
+  r.kernel = kGeneral;
+  const int forced = forced_kernel_of(true);
+  if (forced == kGeneral || tuning(DX_TUNE_ATTN_SPLITS) != 0) return DX_OK;
+  if (c.dtype == DX_F32) {
+    const int form = forced == kF32Eight ? 8 : forced == kF32Four ? 4 : forced == kF32Pair ? 2 : 0;
+    r.pf = plan_f32(c.B, c.Lq, c.Lk, c.H, c.D, c.cache_len, c.cache_lens, c.n_blocks, c.causal,
+                    cus, form);
+    if (r.pf.fits)
+      r.kernel = r.pf.waves == 8 ? kF32Eight : r.pf.qt == 2 ? kF32Pair : kF32Four;
+  } else if (c.D == 256 &&
+             (forced == kWide || wide_fits(c.B, c.Lq, c.Lk, c.H, c.cache_len, c.cache_lens,
+                                           c.n_blocks, c.causal, cus))) {
+    r.kernel = kWide;
+  }
+  return DX_OK;
 }
 
 template <int D, typename T, int NS>
@@ -3864,7 +3936,7 @@ int attention_entry(const void* q, int64_t q_sb, int64_t q_sl, int64_t q_sh, con
                (long long)D);
   // bf16/f16 at head dim 64 or 128 take the MFMA kernels of this file; fp32
   // and the other head dims take the general kernel (attn_any.hip).
-  const bool general = dtype == DX_F32 || (D != 64 && D != 128);
+  const bool general = general_call(dtype, D);
   const int64_t es = dtype == DX_F32 ? 4 : 2;
   DX_CHECK_ARG(B >= 0 && Lq >= 0 && Lk >= 0 && H > 0, "attention: bad shape");
   DX_CHECK_ARG(Hkv > 0 && H % Hkv == 0,
@@ -3919,22 +3991,13 @@ int attention_entry(const void* q, int64_t q_sb, int64_t q_sl, int64_t q_sh, con
                  (long long)stride);
   }
   if (B * Lq == 0) return DX_OK;
-  Plan p{};
-  AnyPlan pa{};
-  int64_t need;
-  if (!general) {
-    p = make_plan(B, Lq, Lk, H, D, cache_len, cache_lens);
-    DX_CHECK_ARG(p.items < (int64_t(1) << 31), "attention: grid too large");
-    need = p.ws_bytes;
-  } else {
-    // The workspace query takes no dtype: at head dims 64 and 128 it reports
-    // the 16-bit kernels' bytes, and fp32 calls split no more than fits them.
-    const int64_t cap =
-        D == 64 || D == 128 ? make_plan(B, Lq, Lk, H, D, cache_len, cache_lens).ws_bytes : -1;
-    pa = plan_any(B, Lq, Lk, H, D, max_cache, cap, device_cus());
-    DX_CHECK_ARG(pa.items < (int64_t(1) << 31), "attention: grid too large");
-    need = pa.ws_bytes;
-  }
+  Route r;
+  const int routed = route_call(
+      {dtype, B, Lq, Lk, H, D, cache_len, cache_lens, n_blocks, causal != 0, q_sl}, r);
+  if (routed != DX_OK) return routed;
+  const Plan& p = r.p;
+  const AnyPlan& pa = r.pa;
+  const int64_t need = r.ws_bytes;
   if (need > 0 && from_scratch) {
     if (need > kScratchBytes) {
       set_error("attention (no-alloc): this call needs %lld bytes of workspace, more than the "
@@ -3954,7 +4017,6 @@ int attention_entry(const void* q, int64_t q_sb, int64_t q_sl, int64_t q_sh, con
     }
     DX_CHECK_ARG(al16(workspace), "attention: workspace must be 16-byte aligned");
   }
-  if (!general) use_wave_kernel(p, B, Lq, Lk, H, D, cache_len, n_blocks, causal != 0);
   if (general) {
     AttnArgs a{};
     a.q = static_cast<const uint16_t*>(q); a.q_sb = q_sb; a.q_sl = q_sl; a.q_sh = q_sh;
@@ -3986,18 +4048,9 @@ int attention_entry(const void* q, int64_t q_sb, int64_t q_sl, int64_t q_sh, con
     a.n_seg = cache_lens ? int(B) : 0;
     for (int64_t i = 0; cache_lens && i < B; ++i) a.seg_cache[i] = int(cache_lens[i]);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // The kernels of attn_f32.hip and attn_wide.hip where they are the faster
-    // ones; a forced split count keeps the general kernel.
-    const bool free_form = tuning(DX_TUNE_ATTN_SPLITS) == 0;
-    F32Plan pf{};
-    if (dtype == DX_F32 && free_form)
-      pf = plan_f32(B, Lq, Lk, H, D, cache_len, cache_lens, n_blocks, causal != 0, device_cus());
-    const bool wide = D == 256 && dtype != DX_F32 && free_form &&
-                      wide_fits(B, Lq, Lk, H, cache_len, cache_lens, n_blocks, causal != 0,
-                                device_cus());
-    const hipError_t e = pf.fits ? launch_f32(a, int(D), pf, st)
-                         : wide  ? launch_wide(a, dtype, st)
-                                 : launch_any(a, dtype, int(D), pa, st);
+    const hipError_t e = r.kernel == kGeneral ? launch_any(a, dtype, int(D), pa, st)
+                         : r.kernel == kWide  ? launch_wide(a, dtype, st)
+                                              : launch_f32(a, int(D), r.pf, st);
     if (e != hipSuccess) {
       set_error("attention: launch failed: %s", hipGetErrorString(e));
       return DX_ELAUNCH;
@@ -4220,6 +4273,24 @@ extern "C" int64_t dx_attention_workspace_bytes(int64_t B, int64_t Lq, int64_t L
   // kernel's, whatever the dtype.
   if (D == 64 || D == 128) return make_plan(B, Lq, Lk, H, D, cache_len, cache_lens).ws_bytes;
   return plan_any(B, Lq, Lk, H, D, max_cache, -1, device_cus()).ws_bytes;
+}
+
+extern "C" int dx_attention_kernel(int dtype, int64_t B, int64_t Lq, int64_t Lk, int64_t H,
+                                   int64_t D, int64_t cache_len, const int64_t* cache_lens,
+                                   int64_t n_blocks, int causal, int64_t q_sl) {
+  bool ok = (dtype == DX_BF16 || dtype == DX_F16 || dtype == DX_F32) && any_head_dim(D) &&
+            B >= 0 && Lq >= 0 && Lk >= 0 && H > 0 && cache_len >= 0 && n_blocks >= 0 &&
+            !(cache_lens && B > kMaxSeg);
+  for (int64_t i = 0; ok && cache_lens && i < B; ++i) ok = cache_lens[i] >= 0;
+  if (!ok) {
+    set_error("attention_kernel: bad shape");
+    return -DX_EINVAL;
+  }
+  if (B * Lq == 0) return 0;
+  Route r;
+  const int rc = route_call(
+      {dtype, B, Lq, Lk, H, D, cache_len, cache_lens, n_blocks, causal != 0, q_sl}, r);
+  return rc == DX_OK ? r.kernel : -rc;
 }
 
 #ifdef DX_TIMELINE

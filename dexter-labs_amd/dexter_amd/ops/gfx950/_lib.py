@@ -16,7 +16,7 @@ import torch
 
 LIB_NAME = "libdexter_gfx950.so"
 LIB_PATH = Path(__file__).resolve().parents[2] / LIB_NAME
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 DX_OK, DX_EINVAL, DX_ELAUNCH, DX_EFULL, DX_EWORKSPACE = 0, 1, 2, 3, 4
 DX_BF16, DX_F16, DX_F32, DX_I32, DX_I64 = 0, 1, 2, 3, 4
@@ -139,6 +139,8 @@ _SIGNATURES: dict[str, tuple[type, list]] = {
         _f, _i, _p]),
     "dx_attention_workspace_bytes": (_l, [_l, _l, _l, _l, _l, _l,
                                           ctypes.POINTER(ctypes.c_int64)]),
+    "dx_attention_kernel": (_i, [_i, _l, _l, _l, _l, _l, _l,  # dtype, B, Lq, Lk, H, D, cache_len
+                                 ctypes.POINTER(ctypes.c_int64), _l, _i, _l]),  # n_blocks, causal, q_sl
     "dx_qkv_norm_rope": (_i, [
         _p, _l, _l, _i,            # x, sb, sl, io dtype
         _p, _p, _p, _l,            # wq, wk, wv, weight row stride

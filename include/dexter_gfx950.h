@@ -79,7 +79,7 @@ const char* dx_last_error(void);
 
 /* ABI revision of this header; the Python loader checks it. */
 int dx_abi_version(void);
-#define DX_ABI_VERSION 11
+#define DX_ABI_VERSION 12
 
 /*
  * Launch-schedule overrides, for measurement and tests only: process-wide,
@@ -89,7 +89,12 @@ int dx_abi_version(void);
  *   DX_TUNE_ATTN_SPLITS  key splits per attention work item (1..16)
  *   DX_TUNE_ATTN_KERNEL  attention kernel: 1 single-stream, 2 dual-stream
  *                        with a separate merge kernel, 3 paired prefill,
- *                        4 one-launch decode, 5 wave-split (small calls)
+ *                        4 one-launch decode, 5 wave-split (small calls);
+ *                        of the general calls (fp32, or D 16, 32, 256): 6 the
+ *                        general kernel, 7 the 128-query one (16-bit, D 256),
+ *                        8 and 9 the fp32 one with eight and four waves, 10
+ *                        with two query tiles. Calls of the other class, and
+ *                        general calls without that form, are not affected
  *   DX_TUNE_NORM_WAVES   waves per row of the adaLN / gated-residual kernels (1..16)
  *   DX_TUNE_QKV_SPLITS   K splits of the fused QKV GEMM (1..16)
  *   DX_TUNE_QKV_WAVES    fused QKV GEMM form: 0 the LDS-DMA form (waves of 64
@@ -361,6 +366,18 @@ int dx_qk_norm_rope_append_dev(const void* q, int64_t q_sb, int64_t q_sl, int64_
 int64_t dx_attention_workspace_bytes(int64_t B, int64_t Lq, int64_t Lk, int64_t H,
                                      int64_t D, int64_t cache_len,
                                      const int64_t* cache_lens);
+
+/*
+ * The kernel that an attention call of this shape takes on the current device
+ * under the present overrides, as the DX_TUNE_ATTN_KERNEL value that forces
+ * it; 0 for a call without queries. For measurement and tests: no call depends
+ * on it. cache_lens as for dx_attention_workspace_bytes; n_blocks 0: no block
+ * boundaries; q_sl: q's row stride in elements. Returns a negative DX_E* code
+ * on a bad shape. No reference counterpart.
+ */
+int dx_attention_kernel(int dtype, int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D,
+                        int64_t cache_len, const int64_t* cache_lens, int64_t n_blocks,
+                        int causal, int64_t q_sl);
 
 /*
  * QKV projection of a decode chunk fused with the QK-RMSNorm + rotary

@@ -93,3 +93,18 @@ def assert_within_ulp(got, ref, ulps=1, frac=0.999, min_abs=1.0, mean_abs=MEAN_A
         f"{ulps} bf16 ulp (>= {frac}), max {n_ulp[sel].max().item():.1f} ulp there, "
         f"mean-abs {mn:.3e} (<= {mean_abs})")
     return within
+
+
+def attention_kernel(dtype, b, lq, lk, h, d, cache_len=0, lens=None, n_blocks=0, causal=False,
+                     q_sl=None):
+    """The kernel an attention call takes, as the DX_TUNE_ATTN_KERNEL value that forces it."""
+    import ctypes
+
+    from dexter_amd.ops.gfx950 import _lib
+    arr = (ctypes.c_int64 * b)(*lens) if lens is not None else None
+    return _lib.load().dx_attention_kernel(_lib.dtype_code(dtype), b, lq, lk, h, d, cache_len, arr,
+                                           n_blocks, int(causal), h * d if q_sl is None else q_sl)
+
+
+# What attention_kernel reports.
+SINGLE, DUAL, PAIRED, DECODE, WAVE, GENERAL, WIDE, F32_EIGHT, F32_FOUR, F32_PAIR = range(1, 11)

@@ -11,8 +11,12 @@ import re
 from pathlib import Path
 
 import pytest
+import torch
 
 from dexter_amd.ops.gfx950 import _lib
+
+from _util import (DUAL, F32_EIGHT, F32_FOUR, F32_PAIR, GENERAL, PAIRED, SINGLE, WAVE, WIDE,
+                   attention_kernel)
 
 HEADER = Path(__file__).resolve().parents[1] / "include" / "dexter_gfx950.h"
 
@@ -202,3 +206,27 @@ def test_general_kernel_plan(built_lib):
     rc = lib.dx_blockwise_causal_attention(*args, 7, 1, 8, 8, 2, 2, 64, 0, None,
                                            _lib.DX_I32, 0, 0, 1.0, None, 0, None)
     assert rc == _lib.DX_EINVAL and "dtype code 7" in lib.dx_last_error().decode()
+
+
+def test_kernel_choice(built_lib):
+    """Which kernel a call takes, by shape and by override (256 CUs without a GPU)."""
+    bf, f32 = torch.bfloat16, torch.float32
+    assert attention_kernel(bf, 1, 83, 83, 24, 128, 1245) == DUAL
+    assert attention_kernel(bf, 1, 8192, 8192, 24, 128, n_blocks=8) == PAIRED
+    assert attention_kernel(bf, 1, 300, 300, 16, 128, causal=True) == WAVE
+    assert attention_kernel(bf, 1, 2048, 2048, 16, 256) == WIDE
+    assert attention_kernel(bf, 1, 83, 83, 24, 32, 1245) == GENERAL
+    assert attention_kernel(f32, 1, 332, 332, 24, 128, 996, n_blocks=4) == F32_FOUR
+    assert attention_kernel(f32, 1, 83, 83, 24, 16, 1245) == GENERAL
+    assert attention_kernel(bf, 4, 99, 99, 24, 128, lens=[0, 332, 1245, 3237], n_blocks=2) == DUAL
+    assert attention_kernel(bf, 1, 0, 0, 16, 256) == 0
+    assert attention_kernel(bf, 1, 8, 8, 2, 96) < 0 and attention_kernel(bf, 1, 8, 8, 2, 64, -1) < 0
+    for kernel in range(SINGLE, F32_PAIR + 1):
+        with _lib.tuning(_lib.TUNE_ATTN_KERNEL, kernel):
+            # An override of one class of calls leaves the other's choice alone.
+            mine = attention_kernel(bf, 1, 83, 83, 24, 128, 1245)
+            assert mine == (kernel if kernel <= WAVE else DUAL)
+            wide = attention_kernel(bf, 1, 2048, 2048, 16, 256)
+            assert wide == (GENERAL if kernel == GENERAL else WIDE)
+            fp32 = attention_kernel(f32, 1, 332, 332, 24, 128, 996, n_blocks=4)
+            assert fp32 == (kernel if kernel in (GENERAL, F32_EIGHT, F32_PAIR) else F32_FOUR)

@@ -30,7 +30,7 @@ from dexter_amd.bench.workloads import CONFIGS, make_inputs
 from dexter_amd.ops.gfx950 import _lib
 from oracle import attention as oatt
 
-from _util import assert_parity
+from _util import F32_EIGHT, F32_FOUR, F32_PAIR, GENERAL, WIDE, assert_parity, attention_kernel
 
 pytestmark = pytest.mark.gpu
 
@@ -92,12 +92,12 @@ def test_c1_shape_fp32(device, built_lib, splits):
 MODES = ["cache", "causal", "blocks", "blocks_any", "cross"]
 # (dtype, head dim) pairs the general kernel runs: fp32 at any head dim, 16-bit
 # types at those the MFMA kernels do not take.
-GENERAL = [(dt, d) for dt in (torch.float32, torch.bfloat16, torch.float16)
-           for d in (16, 32, 64, 256) if dt == torch.float32 or d != 64]
+GENERAL_TYPES = [(dt, d) for dt in (torch.float32, torch.bfloat16, torch.float16)
+                 for d in (16, 32, 64, 256) if dt == torch.float32 or d != 64]
 
 
-@pytest.mark.parametrize("dtype,d", GENERAL,
-                         ids=[f"{str(dt)[6:]}-D{d}" for dt, d in GENERAL])
+@pytest.mark.parametrize("dtype,d", GENERAL_TYPES,
+                         ids=[f"{str(dt)[6:]}-D{d}" for dt, d in GENERAL_TYPES])
 @pytest.mark.parametrize("mode", MODES)
 def test_head_dims_dtypes_masks(device, built_lib, dtype, d, mode):
     b, lq, h = 2, 77, 4
@@ -230,8 +230,7 @@ def test_general_kernel_leaves_the_counter_region_alone(device, built_lib):
 
 
 # The prefill kernel of head dim 256 (attn_wide.hip: 128 queries per work item, two
-# streams of 32-key tiles) at the edges of its tiles. Enough heads that the planner
-# takes it (a forced split count goes to the general kernel, the other side here).
+# streams of 32-key tiles) at the edges of its tiles, forced, against the general kernel.
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("b,lq,lk,h,hkv,cache_len,mask", [
     (1, 1, 1, 64, 64, 0, None), (1, 33, 33, 64, 8, 0, "causal"), (1, 127, 127, 32, 32, 31, None),
@@ -254,13 +253,17 @@ def test_wide_heads_prefill(device, built_lib, dtype, b, lq, lk, h, hkv, cache_l
     call = lambda: ops.blockwise_causal_attention(  # noqa: E731
         qd, kvd[:, :, 0], kvd[:, :, 1], kv_cache=dev(cache), cache_len=cache_len,
         block_boundaries=dev(bb), causal=causal)
-    got = call()
-    with _lib.tuning(_lib.TUNE_ATTN_SPLITS, 1):
-        general = call()
+    sides = {}
+    for kernel in (WIDE, GENERAL):
+        with _lib.tuning(_lib.TUNE_ATTN_KERNEL, kernel):
+            n_blocks = len(mask) if isinstance(mask, list) else 0
+            assert attention_kernel(dtype, b, lq, lk, h, 256, cache_len, n_blocks=n_blocks,
+                                    causal=causal, q_sl=256) == kernel
+            sides[kernel] = call()
+    got, general = sides[WIDE], sides[GENERAL]
     seen = ~torch.isnan(ref)
     assert torch.equal(torch.isnan(got.cpu()), ~seen)
     assert torch.equal(torch.isnan(general.cpu()), ~seen)
-    assert not torch.equal(got.cpu()[seen], general.cpu()[seen]) or lq * lk == 1
     for what, other in (("oracle", ref), ("general kernel", general.float().cpu())):
         assert_parity(got.cpu()[seen], other[seen], what=f"{what} {lq}x{lk}+{cache_len} {mask}")
 
@@ -284,16 +287,17 @@ def test_wide_heads_scales_cursor_ragged(device, built_lib, scale):
 
 
 # The fp32 kernel that deals 16-key tiles to a workgroup's waves (attn_f32.hip) at the
-# edges of its tiles and in each of its forms (eight waves; four waves past one item per
-# CU; two query tiles per item past 700 items; head dim 256). Bar: fp32 sums in another
+# edges of its tiles and in each of its forms, forced (eight waves; four waves; four waves
+# and two query tiles per item; head dim 256 has four waves and one tile). Bar: fp32 sums in another
 # order, a few 1e-7 of values of size one, as the general kernel's tests.
-@pytest.mark.parametrize("d", [32, 64, 128, 256])
+@pytest.mark.parametrize("d,form", [(d, f) for d in (32, 64, 128)
+                                    for f in (F32_EIGHT, F32_FOUR, F32_PAIR)] + [(256, F32_FOUR)])
 @pytest.mark.parametrize("b,lq,lk,h,hkv,cache_len,mask", [
     (1, 1, 1, 8, 8, 0, None), (1, 17, 17, 24, 3, 15, "causal"), (2, 33, 33, 12, 12, 17, [0, 16, 32]),
     (1, 83, 130, 12, 4, 0, None), (1, 96, 96, 8, 8, 20, [40, 0, 70]), (1, 80, 80, 8, 8, 10, [-30, 20]),
     (1, 100, 100, 48, 48, 40, "causal"), (1, 97, 97, 104, 8, 3, [0, 50]),
 ])
-def test_fp32_wave_split(device, built_lib, d, b, lq, lk, h, hkv, cache_len, mask):
+def test_fp32_wave_split(device, built_lib, d, form, b, lq, lk, h, hkv, cache_len, mask):
     g = torch.Generator().manual_seed(lq + h + d)
     rand = lambda *s: torch.randn(s, generator=g)  # noqa: E731
     q = rand(b, h, lq, d).transpose(1, 2)  # head-major in memory
@@ -308,9 +312,14 @@ def test_fp32_wave_split(device, built_lib, d, b, lq, lk, h, hkv, cache_len, mas
     call = lambda: ops.blockwise_causal_attention(  # noqa: E731
         qd, kvd[:, :, 0], kvd[:, :, 1], kv_cache=dev(cache), cache_len=cache_len,
         block_boundaries=dev(bb), causal=causal)
-    got = call()
-    with _lib.tuning(_lib.TUNE_ATTN_SPLITS, 1):
-        general = call()
+    sides = {}
+    for kernel in (form, GENERAL):
+        with _lib.tuning(_lib.TUNE_ATTN_KERNEL, kernel):
+            n_blocks = len(mask) if isinstance(mask, list) else 0
+            assert attention_kernel(torch.float32, b, lq, lk, h, d, cache_len, n_blocks=n_blocks,
+                                    causal=causal, q_sl=d) == kernel
+            sides[kernel] = call()
+    got, general = sides[form], sides[GENERAL]
     seen = ~torch.isnan(ref)
     assert torch.equal(torch.isnan(got.cpu()), ~seen)
     for what, other in (("oracle", ref), ("general kernel", general.cpu())):
