@@ -3786,7 +3786,7 @@ int route_call(const CallShape& c, Route& r) {
                     cus, form);
     if (r.pf.fits)
       r.kernel = r.pf.waves == 8 ? kF32Eight : r.pf.qt == 2 ? kF32Pair : kF32Four;
-  } else if (c.D == 256 &&
+  } else if (c.D == 256 && q_rows_fit(std::min<int64_t>(c.Lq, kWideQ), c.q_sl, c.D) &&
              (forced == kWide || wide_fits(c.B, c.Lq, c.Lk, c.H, c.cache_len, c.cache_lens,
                                            c.n_blocks, c.causal, cus))) {
     r.kernel = kWide;

@@ -32,7 +32,7 @@ namespace dx {
 namespace {
 
 constexpr int kD = 256, kKS = kD / 16, kDT = kD / 32, kRB = 2 * kD;
-constexpr int kWideQ = 128, kWideN = 32;     // queries per item, keys per tile
+constexpr int kWideN = 32;                   // keys per tile
 constexpr int kTileB = kWideN * kRB;         // bytes of a K or V tile
 constexpr int kStageB = 2 * kTileB;
 constexpr int kStreamB = 2 * kStageB;        // two stages
@@ -66,11 +66,12 @@ __global__ __launch_bounds__(512, 1) void attn_wide_kernel(AttnArgs a) {
   const uint32_t kcol = uint32_t(n ^ swz_k(lr)), vcol = uint32_t(n ^ (4 * swz_v(lr)));
 
   // Q: rows 0..63 into stream 0's second stage, 64..127 into stream 1's (64
-  // pieces, eight per wave); rows past Lq read as zeros.
+  // pieces, eight per wave); rows past Lq read as zeros. The descriptor covers
+  // this item's rows only (q_rows_fit): all of a long q need not fit one.
   {
     const __amdgpu_buffer_rsrc_t rq =
-        make_rsrc(a.q + b * a.q_sb + int64_t(q0) * a.q_sl + h * a.q_sh, a.Lq - q0,
-                  int(a.q_sl) * 2, kD);
+        make_rsrc(a.q + b * a.q_sb + int64_t(q0) * a.q_sl + h * a.q_sh,
+                  min(a.Lq - q0, kWideQ), int(a.q_sl) * 2, kD);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int r = 64 * stream + 8 * i + lr;

@@ -230,3 +230,18 @@ def test_kernel_choice(built_lib):
             assert wide == (GENERAL if kernel == GENERAL else WIDE)
             fp32 = attention_kernel(f32, 1, 332, 332, 24, 128, 996, n_blocks=4)
             assert fp32 == (kernel if kernel in (GENERAL, F32_EIGHT, F32_PAIR) else F32_FOUR)
+
+
+def test_query_rows_past_a_descriptor(built_lib):
+    """Kernels that fetch a work item's query rows through one buffer descriptor (2^31 bytes)
+    take every call whose items fit it, however long q is, and no other."""
+    bf = torch.bfloat16
+    last = (2**30 - 1 - 256) // 127  # row stride at which 128 rows of 256 still fit
+    assert attention_kernel(bf, 1, 131136, 32, 64, 256) == WIDE
+    assert attention_kernel(bf, 1, 4096, 32, 64, 256, q_sl=last) == WIDE
+    assert attention_kernel(bf, 1, 4096, 32, 64, 256, q_sl=last + 1) == GENERAL
+    assert attention_kernel(bf, 1, 4096, 32, 64, 256, q_sl=2**40) == GENERAL
+    assert attention_kernel(bf, 1, 4096, 32, 64, 256, q_sl=-256) == GENERAL
+    with _lib.tuning(_lib.TUNE_ATTN_KERNEL, WIDE):
+        assert attention_kernel(bf, 1, 128, 32, 64, 256, q_sl=last + 1) == GENERAL
+        assert attention_kernel(bf, 512, 1, 32, 64, 256, q_sl=2**40) == WIDE  # one row: no stride
