@@ -3026,12 +3026,13 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_wave_kernel(AttnArgs a) {
   const int cache_len = it.cache_len;
   const uint32_t smem_b = lds_addr(smem);
 
-  // Q rows into LDS first (whole-row pieces; rows past Lq read as zeros).
+  // Q rows into LDS first (whole-row pieces; rows past Lq read as zeros). The
+  // descriptor covers this item's rows only (q_rows_fit).
   const int lr = lane / CR, lx = lane % CR;  // this lane's row within a piece, physical chunk
   {
     const __amdgpu_buffer_rsrc_t rq =
-        make_rsrc(a.q + b * a.q_sb + int64_t(q0) * a.q_sl + h * a.q_sh, a.Lq - q0,
-                  int(a.q_sl) * 2, D);
+        make_rsrc(a.q + b * a.q_sb + int64_t(q0) * a.q_sl + h * a.q_sh,
+                  min(a.Lq - q0, kWaveQ), int(a.q_sl) * 2, D);
     for (int p = wid; p < kWaveQ / RPP; p += NW) {
       const int r = p * RPP + lr;
       const uint32_t o = uint32_t(r) * uint32_t(a.q_sl) * 2 + uint32_t(16 * (lx ^ L::kswz(r)));
@@ -3761,7 +3762,8 @@ int route_call(const CallShape& c, Route& r) {
     r.p = make_plan(c.B, c.Lq, c.Lk, c.H, c.D, c.cache_len, c.cache_lens);
     DX_CHECK_ARG(r.p.items < (int64_t(1) << 31), "attention: grid too large");
     r.ws_bytes = r.p.ws_bytes;
-    use_wave_kernel(r.p, c.B, c.Lq, c.Lk, c.H, c.D, c.cache_len, c.n_blocks, c.causal);
+    if (q_rows_fit(std::min<int64_t>(c.Lq, kWaveQ), c.q_sl, c.D))
+      use_wave_kernel(r.p, c.B, c.Lq, c.Lk, c.H, c.D, c.cache_len, c.n_blocks, c.causal);
     r.kernel = r.p.kernel;
     return DX_OK;
   }

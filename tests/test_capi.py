@@ -245,3 +245,6 @@ def test_query_rows_past_a_descriptor(built_lib):
     with _lib.tuning(_lib.TUNE_ATTN_KERNEL, WIDE):
         assert attention_kernel(bf, 1, 128, 32, 64, 256, q_sl=last + 1) == GENERAL
         assert attention_kernel(bf, 512, 1, 32, 64, 256, q_sl=2**40) == WIDE  # one row: no stride
+    last = (2**30 - 1 - 128) // 31
+    assert attention_kernel(bf, 1, 300, 300, 16, 128, causal=True, q_sl=last) == WAVE
+    assert attention_kernel(bf, 1, 300, 300, 16, 128, causal=True, q_sl=last + 1) == DUAL

@@ -9,7 +9,7 @@ import torch
 import dexter_amd.ops as ops
 from oracle import attention as oatt
 
-from _util import GENERAL, WIDE, assert_parity, attention_kernel
+from _util import DUAL, GENERAL, WAVE, WIDE, assert_parity, attention_kernel
 
 pytestmark = pytest.mark.gpu
 
@@ -47,5 +47,23 @@ def test_wide_heads_item_past_a_descriptor(device, built_lib):
     h, d, lq, lk = 32, 256, 130, 64
     step = _step(128, 2**31)
     assert attention_kernel(torch.bfloat16, 1, lq, lk, h, d, q_sl=step) == GENERAL
+    k, v = (torch.randn(1, lk, h, d, device=device, dtype=torch.bfloat16) for _ in range(2))
+    _check(_strided(device, lq, h, d, step), k, v, list(range(lq)))
+
+
+def test_wave_split(device, built_lib):
+    """A q view whose 200 rows span 4 GiB."""
+    h, d, lq, lk = 16, 128, 200, 64
+    step = _step(lq, 2**32)
+    assert attention_kernel(torch.bfloat16, 1, lq, lk, h, d, q_sl=step) == WAVE
+    k, v = (torch.randn(1, lk, h, d, device=device, dtype=torch.bfloat16) for _ in range(2))
+    _check(_strided(device, lq, h, d, step), k, v, list(range(lq)))
+
+
+def test_wave_split_item_past_a_descriptor(device, built_lib):
+    """32 rows over 2 GiB: the kernel that the call had without the wave split."""
+    h, d, lq, lk = 16, 128, 40, 256
+    step = _step(32, 2**31)
+    assert attention_kernel(torch.bfloat16, 1, lq, lk, h, d, q_sl=step) == DUAL
     k, v = (torch.randn(1, lk, h, d, device=device, dtype=torch.bfloat16) for _ in range(2))
     _check(_strided(device, lq, h, d, step), k, v, list(range(lq)))
