@@ -2088,8 +2088,9 @@ __global__ __launch_bounds__(64 * kPairWaves, 1) void attn_pair_kernel(AttnArgs 
   const uint32_t smem_b = lds_addr(smem);
   // The work item's Q rows into the row area (rows past Lq read as zeros),
   // then K_0 into stage 0 and V of step -1 (nothing: zeros) into V stage 2.
+  // The descriptor covers these rows only (q_rows_fit).
   Rows::load_q(make_rsrc(a.q + b * a.q_sb + int64_t(q0) * a.q_sl + h * a.q_sh,
-                         max(a.Lq - q0, 0), int(a.q_sl) * 2, D),
+                         min(a.Lq - q0, kBMPair), int(a.q_sl) * 2, D),
                int(a.q_sl) * 2, a.Lq - q0, smem_b + Rows::off, wid, lane);
   Dma dma;
   dma.init(wid, lane, src);
@@ -3666,6 +3667,23 @@ Plan make_plan(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_t 
   return p;
 }
 
+// Turn a plan into one launch of `kernel` with unsplit work items of bm
+// queries. The workspace the call has to bring is unchanged (its query knows
+// neither the mask nor the strides); the launch leaves it untouched.
+void one_launch(Plan& p, int kernel, int bm, int64_t B, int64_t Lq, int64_t H) {
+  p.kernel = kernel;
+  p.bm = p.prow = bm;
+  p.n_qtiles = int(cdiv(Lq, bm));
+  p.items = B * H * p.n_qtiles;
+  p.uniform_splits = 1;
+  for (size_t k = 0; k < p.seg_splits.size(); ++k) {
+    p.seg_splits[k] = 1;
+    p.seg_base[k + 1] = int(int64_t(k + 1) * H * p.n_qtiles);
+  }
+  p.partials = p.comb_blocks = p.counter_bytes = p.ws_bytes = 0;
+  p.pmerge = p.spread = false;
+}
+
 // Whether a call goes to attn_wave_kernel, by its work items I (32 queries of
 // a head) and the mean key tiles T of 32 an item visits (causal and blocks: an
 // item sees about half of the new keys' tiles).
@@ -3692,8 +3710,7 @@ bool wave_kernel_fits(double items, double tiles, int64_t D, int64_t nb, bool ca
 }
 
 // Turn the plan of a call that wave_kernel_fits into one launch of
-// attn_wave_kernel. The workspace the call has to bring is unchanged (the
-// workspace query knows no mask); this kernel leaves it untouched.
+// attn_wave_kernel.
 void use_wave_kernel(Plan& p, int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D,
                      int64_t cache_len, int64_t n_blocks, bool causal) {
   const int forced = forced_kernel_of(false);
@@ -3719,18 +3736,8 @@ void use_wave_kernel(Plan& p, int64_t B, int64_t Lq, int64_t Lk, int64_t H, int6
   }
   if (items >= (int64_t(1) << 31)) return;  // past the grid's limit
   if (!forced && !wave_kernel_fits(double(items), tiles, D, n_blocks, causal, cus)) return;
-  p.kernel = kWave;
   p.nqw = items <= cus ? 8 : 4;
-  p.bm = kWaveQ;
-  p.n_qtiles = int(n_qtiles);
-  p.items = items;
-  p.uniform_splits = 1;
-  for (size_t k = 0; k < p.seg_splits.size(); ++k) {
-    p.seg_splits[k] = 1;
-    p.seg_base[k + 1] = int(int64_t(k + 1) * H * n_qtiles);
-  }
-  p.partials = p.comb_blocks = p.counter_bytes = p.ws_bytes = 0;
-  p.pmerge = p.spread = false;
+  one_launch(p, kWave, kWaveQ, B, Lq, H);
 }
 
 // fp32 inputs and the other head dims take the general kernels.
@@ -3762,6 +3769,11 @@ int route_call(const CallShape& c, Route& r) {
     r.p = make_plan(c.B, c.Lq, c.Lk, c.H, c.D, c.cache_len, c.cache_lens);
     DX_CHECK_ARG(r.p.items < (int64_t(1) << 31), "attention: grid too large");
     r.ws_bytes = r.p.ws_bytes;
+    // Items whose query rows lie outside one descriptor: the single-stream
+    // kernel, which reads q by pointer.
+    if ((r.p.kernel == kPaired || r.p.kernel == kDecode) &&
+        !q_rows_fit(std::min<int64_t>(c.Lq, r.p.bm), c.q_sl, c.D))
+      one_launch(r.p, kSingle, kBM, c.B, c.Lq, c.H);
     if (q_rows_fit(std::min<int64_t>(c.Lq, kWaveQ), c.q_sl, c.D))
       use_wave_kernel(r.p, c.B, c.Lq, c.Lk, c.H, c.D, c.cache_len, c.n_blocks, c.causal);
     r.kernel = r.p.kernel;

@@ -15,7 +15,7 @@ import torch
 
 from dexter_amd.ops.gfx950 import _lib
 
-from _util import (DUAL, F32_EIGHT, F32_FOUR, F32_PAIR, GENERAL, PAIRED, SINGLE, WAVE, WIDE,
+from _util import (DECODE, DUAL, F32_EIGHT, F32_FOUR, F32_PAIR, GENERAL, PAIRED, SINGLE, WAVE, WIDE,
                    attention_kernel)
 
 HEADER = Path(__file__).resolve().parents[1] / "include" / "dexter_gfx950.h"
@@ -248,3 +248,10 @@ def test_query_rows_past_a_descriptor(built_lib):
     last = (2**30 - 1 - 128) // 31
     assert attention_kernel(bf, 1, 300, 300, 16, 128, causal=True, q_sl=last) == WAVE
     assert attention_kernel(bf, 1, 300, 300, 16, 128, causal=True, q_sl=last + 1) == DUAL
+    last = (2**30 - 1 - 128) // 255
+    assert attention_kernel(bf, 1, 262272, 64, 64, 128) == PAIRED
+    assert attention_kernel(bf, 1, 300, 1000, 48, 128, q_sl=last) == PAIRED
+    assert attention_kernel(bf, 1, 300, 1000, 48, 128, q_sl=last + 1) == SINGLE
+    with _lib.tuning(_lib.TUNE_ATTN_KERNEL, DECODE):  # 96 rows
+        assert attention_kernel(bf, 1, 300, 1000, 48, 128, q_sl=last + 1) == DECODE
+        assert attention_kernel(bf, 1, 300, 1000, 48, 128, q_sl=4 * last) == SINGLE
