@@ -3494,7 +3494,8 @@ Plan make_plan(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_t 
                const int64_t* cache_lens) {
   Plan p{};
   const int cus = device_cus();
-  const int forced_kernel = forced_kernel_of(false);
+  // The wave split is put over a call's own plan (use_wave_kernel), forced or not.
+  const int forced = forced_kernel_of(false), forced_kernel = forced == kWave ? 0 : forced;
   const int forced_splits = tuning(DX_TUNE_ATTN_SPLITS);
   // Segments: one per sequence of a ragged batch, longest first; a uniform
   // call is one segment of all B*H (batch, head) pairs.

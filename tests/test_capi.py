@@ -248,6 +248,8 @@ def test_query_rows_past_a_descriptor(built_lib):
     last = (2**30 - 1 - 128) // 31
     assert attention_kernel(bf, 1, 300, 300, 16, 128, causal=True, q_sl=last) == WAVE
     assert attention_kernel(bf, 1, 300, 300, 16, 128, causal=True, q_sl=last + 1) == DUAL
+    with _lib.tuning(_lib.TUNE_ATTN_KERNEL, WAVE):  # forced, it falls back to the same plan
+        assert attention_kernel(bf, 1, 300, 300, 16, 128, causal=True, q_sl=last + 1) == DUAL
     last = (2**30 - 1 - 128) // 255
     assert attention_kernel(bf, 1, 262272, 64, 64, 128) == PAIRED
     assert attention_kernel(bf, 1, 300, 1000, 48, 128, q_sl=last) == PAIRED
