@@ -203,6 +203,12 @@ AnyPlan plan_any(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_
 // n_seg == B > 0. dtype: DX_BF16, DX_F16 or DX_F32.
 hipError_t launch_any(const AttnArgs& a, int dtype, int D, const AnyPlan& p, hipStream_t st);
 
+// Whether a one-dimensional grid can be launched: HIP takes less than 2^31
+// workgroups and less than 2^32 threads.
+inline bool grid_fits(int64_t blocks, int64_t threads) {
+  return blocks < (int64_t(1) << 31) && blocks * threads < (int64_t(1) << 32);
+}
+
 // Whether the query rows of a work item (16-bit, `rows` at most, D elements
 // each, q_sl elements apart) lie within one buffer descriptor: its record count
 // and the byte offsets into it stay below 2^31. The descriptor starts at the
@@ -213,9 +219,10 @@ inline bool q_rows_fit(int64_t rows, int64_t q_sl, int64_t D) {
 }
 
 // Head dim 256, 16-bit inputs, one launch without key splits (attn_wide.hip);
-// a as for launch_any. kWideQ: queries per work item. wide_fits: whether it is
+// a as for launch_any. kWideQ: queries per work item, one to a
+// workgroup. wide_fits: whether it is
 // the faster one for sequences with these cache lengths.
-constexpr int kWideQ = 128;
+constexpr int kWideQ = 128, kWideThreads = 512;
 bool wide_fits(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t cache_len,
                const int64_t* cache_lens, int64_t n_blocks, bool causal, int cus);
 hipError_t launch_wide(AttnArgs a, int dtype, hipStream_t st);

@@ -318,7 +318,6 @@ F32Plan plan_f32(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_
   F32Plan p{};
   if (D < 32) return p;
   const int64_t items = B * H * ((Lq + 15) / 16);
-  if (items >= (int64_t(1) << 31)) return p;
   const bool many = D < 256 && items > 700;
   p.waves = D < 256 && items <= cus ? 8 : 4;
   p.qt = many ? 2 : 1;
@@ -326,6 +325,8 @@ F32Plan plan_f32(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_
     p.waves = D < 256 && form == 8 ? 8 : 4;
     p.qt = D < 256 && form == 2 ? 2 : 1;
   }
+  const int64_t blocks = B * H * ((Lq + 16 * p.qt - 1) / (16 * p.qt));
+  if (!grid_fits(blocks, 64 * p.waves)) return p;
   p.fits = many || form;
   if (p.fits) return p;
   auto tiles = [](int64_t keys) { return double((keys + kKeys - 1) / kKeys); };

@@ -3735,9 +3735,10 @@ void use_wave_kernel(Plan& p, int64_t B, int64_t Lq, int64_t Lk, int64_t H, int6
     }
     if (!forced && double(longest) + seen > 20) return;
   }
-  if (items >= (int64_t(1) << 31)) return;  // past the grid's limit
   if (!forced && !wave_kernel_fits(double(items), tiles, D, n_blocks, causal, cus)) return;
-  p.nqw = items <= cus ? 8 : 4;
+  const int waves = items <= cus ? 8 : 4;
+  if (!grid_fits(items, 64 * waves)) return;
+  p.nqw = waves;
   one_launch(p, kWave, kWaveQ, B, Lq, H);
 }
 
@@ -3802,6 +3803,7 @@ int route_call(const CallShape& c, Route& r) {
     if (r.pf.fits)
       r.kernel = r.pf.waves == 8 ? kF32Eight : r.pf.qt == 2 ? kF32Pair : kF32Four;
   } else if (c.D == 256 && q_rows_fit(std::min<int64_t>(c.Lq, kWideQ), c.q_sl, c.D) &&
+             grid_fits(c.B * c.H * cdiv(c.Lq, kWideQ), kWideThreads) &&
              (forced == kWide || wide_fits(c.B, c.Lq, c.Lk, c.H, c.cache_len, c.cache_lens,
                                            c.n_blocks, c.causal, cus))) {
     r.kernel = kWide;

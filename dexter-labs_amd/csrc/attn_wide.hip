@@ -44,7 +44,7 @@ __device__ __forceinline__ int swz_k(int r) { return (r & 15) ^ ((r >> 4) & 1); 
 __device__ __forceinline__ int swz_v(int r) { return (r & 3) ^ ((r >> 2) & 1); }
 
 template <typename T>
-__global__ __launch_bounds__(512, 1) void attn_wide_kernel(AttnArgs a) {
+__global__ __launch_bounds__(kWideThreads, 1) void attn_wide_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   prefetch_args(a);
   const AnyItem it = any_item(a, int(blockIdx.x));
@@ -279,7 +279,7 @@ hipError_t launch_wide_t(const AttnArgs& a, hipStream_t st) {
   const hipError_t e = opt_in_lds(fn, kWideLds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((attn_wide_kernel<T>), dim3(unsigned(int64_t(a.B) * a.H * a.n_qtiles)),
-                     dim3(512), kWideLds, st, a);
+                     dim3(kWideThreads), kWideLds, st, a);
   return hipGetLastError();
 }
 
@@ -296,7 +296,6 @@ hipError_t launch_wide_t(const AttnArgs& a, hipStream_t st) {
 bool wide_fits(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t cache_len,
                const int64_t* cache_lens, int64_t n_blocks, bool causal, int cus) {
   const int64_t per_seq = H * ((Lq + kWideQ - 1) / kWideQ), items = B * per_seq;
-  if (items >= (int64_t(1) << 31)) return false;
   if (items > cus) return true;
   auto tiles = [](int64_t keys) { return double((keys + kWideN - 1) / kWideN); };
   double seen = tiles(Lk);  // mean new-key tiles of an item

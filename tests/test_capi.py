@@ -257,3 +257,17 @@ def test_query_rows_past_a_descriptor(built_lib):
     with _lib.tuning(_lib.TUNE_ATTN_KERNEL, DECODE):  # 96 rows
         assert attention_kernel(bf, 1, 300, 1000, 48, 128, q_sl=last + 1) == DECODE
         assert attention_kernel(bf, 1, 300, 1000, 48, 128, q_sl=4 * last) == SINGLE
+
+
+def test_grids_past_the_launch_limit(built_lib):
+    """A launch holds less than 2^32 threads: calls whose finer work items pass that stay on the
+    general kernel, which has fewer of them."""
+    f32, bf = torch.float32, torch.bfloat16
+    assert attention_kernel(f32, 1, 2**23 - 32, 64, 64, 32) == F32_PAIR
+    assert attention_kernel(f32, 1, 2**23, 64, 64, 32) == GENERAL
+    with _lib.tuning(_lib.TUNE_ATTN_KERNEL, WIDE):
+        assert attention_kernel(bf, 1 << 10, 1, 32, (1 << 13) - 1, 256) == WIDE
+        assert attention_kernel(bf, 1 << 10, 1, 32, 1 << 13, 256) == GENERAL
+    with _lib.tuning(_lib.TUNE_ATTN_KERNEL, WAVE):
+        assert attention_kernel(bf, 1 << 11, 1, 32, (1 << 13) - 1, 128) == WAVE
+        assert attention_kernel(bf, 1 << 11, 1, 32, 1 << 13, 128) != WAVE
