@@ -219,12 +219,12 @@ inline bool q_rows_fit(int64_t rows, int64_t q_sl, int64_t D) {
 }
 
 // Head dim 256, 16-bit inputs, one launch without key splits (attn_wide.hip);
-// a as for launch_any. kWideQ: queries per work item, one to a
-// workgroup. wide_fits: whether it is
-// the faster one for sequences with these cache lengths.
+// a as for launch_any. kWideQ: queries per work item, one to a workgroup.
+// wide_fits: whether it is the faster one for sequences with these cache lengths
+// (splits: the key splits that launch_any would take).
 constexpr int kWideQ = 128, kWideThreads = 512;
 bool wide_fits(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t cache_len,
-               const int64_t* cache_lens, int64_t n_blocks, bool causal, int cus);
+               const int64_t* cache_lens, int64_t n_blocks, bool causal, int splits, int cus);
 hipError_t launch_wide(AttnArgs a, int dtype, hipStream_t st);
 
 // fp32 inputs at head dims 32 to 256, keys dealt to a workgroup's waves

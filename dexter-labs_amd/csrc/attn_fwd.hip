@@ -3805,7 +3805,7 @@ int route_call(const CallShape& c, Route& r) {
   } else if (c.D == 256 && q_rows_fit(std::min<int64_t>(c.Lq, kWideQ), c.q_sl, c.D) &&
              grid_fits(c.B * c.H * cdiv(c.Lq, kWideQ), kWideThreads) &&
              (forced == kWide || wide_fits(c.B, c.Lq, c.Lk, c.H, c.cache_len, c.cache_lens,
-                                           c.n_blocks, c.causal, cus))) {
+                                           c.n_blocks, c.causal, r.pa.splits, cus))) {
     r.kernel = kWide;
   }
   return DX_OK;

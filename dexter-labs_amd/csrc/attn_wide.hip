@@ -26,6 +26,8 @@
 
 #include <float.h>
 
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace dx {
@@ -285,29 +287,42 @@ hipError_t launch_wide_t(const AttnArgs& a, hipStream_t st) {
 
 }  // namespace
 
-// Items past one per CU: always. Below, this kernel takes as long as its
-// longest item (9.5 us and 1.04 us per 32-key tile, measured over 24 to 256
-// items), while attn_any16_kernel splits the keys to fill the chip (19.5 us
-// and 9.5 ns per item and tile). Cold, us per call, that kernel -> this one: 16
-// heads x 2048 149 -> 92; 24 heads x 1000 75.6 -> 44.5, causal 56.7 -> 42.0; 16
-// heads x 400 29.4 -> 22.7; 24 heads x 900 onto 512 keys 45.4 -> 28.7; past the
-// line 8 heads x 1000 causal 32.5 -> 40.4, 24 heads x 300 over 2000 cached
-// 59.4 -> 82.0.
+// Modelled times (us) of this kernel and of attn_any16_kernel, by 32-key tiles:
+//  * here: rounds of one workgroup per CU, 9.5 each, and 0.89 a tile of a CU's
+//    items in turn (rounds x the mean item, or the longest one), up to 1.4
+//    where every CU has work throughout;
+//  * there: 7.6 (16.3 when it splits the keys and merges), 6 ns per tile of
+//    every 64-query item, and 12 ns per item for its queries and results.
+// Measured over 1 to 128 sequences, 1 to 32,768 queries and 16 to 8,000 keys
+// (cold, us per call, that kernel -> this one). Here: 16 heads x 2048 155 -> 91;
+// 24 heads x 1000 81 -> 48, causal 59 -> 46; 16 heads x 400 31 -> 23; 64 heads
+// x 8192 over 128 keys 226 -> 209; 8 x 16 heads, 200 over 2000 160 -> 101; 32 x
+// 16 heads, 83 over 8000 1376 -> 699. There: 8 heads x 1000 causal 34 -> 41, 24
+// heads x 300 over 2000 57 -> 84; 8 x 16 heads, 64 over 8000 209 -> 278; 17 x 16
+// heads, 16 over 500 49 -> 63 and 64 over 8000 497 -> 591; 64 x 16 heads, 1 over
+// 100 36 -> 53. Wrong by more than 3% at three of 165: 8 x 16 heads, 16 over 500
+// (30 for 29), and 40 x 16 heads (4 K/V) over 4000, 1 query (398 for 353) and 32
+// (402 for 378).
 bool wide_fits(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t cache_len,
-               const int64_t* cache_lens, int64_t n_blocks, bool causal, int cus) {
-  const int64_t per_seq = H * ((Lq + kWideQ - 1) / kWideQ), items = B * per_seq;
-  if (items > cus) return true;
+               const int64_t* cache_lens, int64_t n_blocks, bool causal, int splits, int cus) {
   auto tiles = [](int64_t keys) { return double((keys + kWideN - 1) / kWideN); };
   double seen = tiles(Lk);  // mean new-key tiles of an item
   if (causal) seen = (seen + 1) / 2;
   else if (n_blocks > 1) seen *= double(n_blocks + 1) / double(2 * n_blocks);
-  double longest = 0, all = 0;
-  for (int64_t i = 0; i < B; ++i) {
+  double longest = 0, mean = 0;
+  for (int64_t i = 0; i < (cache_lens ? B : 1); ++i) {
     const double c = tiles(cache_lens ? cache_lens[i] : cache_len);
-    longest = c > longest ? c : longest;
-    all += double(per_seq) * (c + seen);
+    longest = std::max(longest, c);
+    mean += (c + seen) / double(cache_lens ? B : 1);
   }
-  return 9.5 + 1.04 * (longest + tiles(Lk)) <= 19.5 + 0.0095 * all;
+  longest += tiles(Lk);
+  const double items = double(B * H * ((Lq + kWideQ - 1) / kWideQ));
+  const double rounds = std::ceil(items / cus), serial = std::max(longest, rounds * mean);
+  const double here = 9.5 * rounds + (0.89 + 0.51 * items * mean / (cus * serial)) * serial;
+  const int64_t tiles64 = (Lq + 63) / 64;
+  const double there = (splits > 1 ? 16.3 : 7.6) +
+                       double(B * H) * (0.006 * double(tiles64) * mean + 0.012 * double(Lq) / 64);
+  return here <= there;
 }
 
 hipError_t launch_wide(AttnArgs a, int dtype, hipStream_t st) {

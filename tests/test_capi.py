@@ -237,11 +237,11 @@ def test_query_rows_past_a_descriptor(built_lib):
     take every call whose items fit it, however long q is, and no other."""
     bf = torch.bfloat16
     last = (2**30 - 1 - 256) // 127  # row stride at which 128 rows of 256 still fit
-    assert attention_kernel(bf, 1, 131136, 32, 64, 256) == WIDE
-    assert attention_kernel(bf, 1, 4096, 32, 64, 256, q_sl=last) == WIDE
-    assert attention_kernel(bf, 1, 4096, 32, 64, 256, q_sl=last + 1) == GENERAL
-    assert attention_kernel(bf, 1, 4096, 32, 64, 256, q_sl=2**40) == GENERAL
-    assert attention_kernel(bf, 1, 4096, 32, 64, 256, q_sl=-256) == GENERAL
+    assert attention_kernel(bf, 1, 131136, 128, 64, 256) == WIDE
+    assert attention_kernel(bf, 1, 4096, 128, 64, 256, q_sl=last) == WIDE
+    assert attention_kernel(bf, 1, 4096, 128, 64, 256, q_sl=last + 1) == GENERAL
+    assert attention_kernel(bf, 1, 4096, 128, 64, 256, q_sl=2**40) == GENERAL
+    assert attention_kernel(bf, 1, 4096, 128, 64, 256, q_sl=-256) == GENERAL
     with _lib.tuning(_lib.TUNE_ATTN_KERNEL, WIDE):
         assert attention_kernel(bf, 1, 128, 32, 64, 256, q_sl=last + 1) == GENERAL
         assert attention_kernel(bf, 512, 1, 32, 64, 256, q_sl=2**40) == WIDE  # one row: no stride
@@ -271,3 +271,21 @@ def test_grids_past_the_launch_limit(built_lib):
     with _lib.tuning(_lib.TUNE_ATTN_KERNEL, WAVE):
         assert attention_kernel(bf, 1 << 11, 1, 32, (1 << 13) - 1, 128) == WAVE
         assert attention_kernel(bf, 1 << 11, 1, 32, 1 << 13, 128) != WAVE
+
+
+def test_head_dim_256_choice_counts_items_and_rounds(built_lib):
+    """Batches of short queries stay on the general kernel, whose items hold 64 queries, also past
+    one 128-query item per CU; prefill-shaped calls go to the 128-query kernel (both measured)."""
+    bf = torch.bfloat16
+    for b, lq, h, cache in [(8, 64, 16, 8000), (8, 16, 16, 2000), (17, 16, 16, 500),
+                            (17, 64, 16, 8000), (12, 64, 24, 2000), (4, 1, 24, 1000),
+                            (1, 300, 24, 2000), (32, 64, 16, 500)]:
+        assert attention_kernel(bf, b, lq, lq, h, 256, cache) == GENERAL, (b, lq, h, cache)
+    for b, lq, h, cache in [(8, 83, 16, 500), (17, 83, 16, 8000), (32, 128, 16, 2000),
+                            (1, 400, 16, 0), (1, 2048, 16, 0), (1, 4100, 16, 0), (2, 1000, 24, 0)]:
+        assert attention_kernel(bf, b, lq, lq, h, 256, cache) == WIDE, (b, lq, h, cache)
+    assert attention_kernel(bf, 1, 1000, 1000, 24, 256, causal=True) == WIDE
+    assert attention_kernel(bf, 1, 1000, 1000, 8, 256, causal=True) == GENERAL
+    # A ragged batch: its longest sequence's items bound the launch.
+    assert attention_kernel(bf, 4, 200, 200, 16, 256, lens=[100, 100, 100, 8000]) == GENERAL
+    assert attention_kernel(bf, 4, 200, 200, 16, 256, lens=[500, 400, 500, 600]) == WIDE

@@ -270,6 +270,11 @@ def test_wide_heads_prefill(device, built_lib, dtype, b, lq, lk, h, hkv, cache_l
 
 @pytest.mark.parametrize("scale", [-0.05, 0.0])
 def test_wide_heads_scales_cursor_ragged(device, built_lib, scale):
+    with _lib.tuning(_lib.TUNE_ATTN_KERNEL, WIDE):
+        _wide_heads_scales_cursor_ragged(device, scale)
+
+
+def _wide_heads_scales_cursor_ragged(device, scale):
     q, k, v = (torch.randn(2, 140, 32, 256, device=device).bfloat16() for _ in range(3))
     cache = torch.randn(2, 2, 100, 32, 256, device=device).bfloat16()
     kw = dict(softmax_scale=scale, block_boundaries=torch.tensor([0, 83], device=device))

@@ -35,7 +35,7 @@ def _step(rows, span):
 
 def test_wide_heads(device, built_lib):
     """64 heads x 256, 131,136 queries: 4 GiB and 2 MB from the first row to the last."""
-    h, d, lq, lk = 64, 256, 131136, 32
+    h, d, lq, lk = 64, 256, 131136, 128
     assert attention_kernel(torch.bfloat16, 1, lq, lk, h, d) == WIDE
     q = torch.randn(1, lq, h, d, device=device, dtype=torch.bfloat16)
     k, v = (torch.randn(1, lk, 16, d, device=device, dtype=torch.bfloat16) for _ in range(2))
@@ -44,7 +44,8 @@ def test_wide_heads(device, built_lib):
 
 def test_wide_heads_item_past_a_descriptor(device, built_lib):
     """A q view with 128 rows over 2 GiB: the general kernel, which reads q by pointer."""
-    h, d, lq, lk = 32, 256, 130, 64
+    h, d, lq, lk = 32, 256, 130, 300
+    assert attention_kernel(torch.bfloat16, 1, lq, lk, h, d) == WIDE
     step = _step(128, 2**31)
     assert attention_kernel(torch.bfloat16, 1, lq, lk, h, d, q_sl=step) == GENERAL
     k, v = (torch.randn(1, lk, h, d, device=device, dtype=torch.bfloat16) for _ in range(2))
