@@ -300,10 +300,12 @@ hipError_t launch_d(const AttnArgs& a, const F32Plan& p, hipStream_t st) {
 }  // namespace
 
 // Form by the 16-query items I: eight waves up to one item per CU; four waves
-// (two workgroups per CU) up to 700; two query tiles per item past that, where
-// there are items enough and K/V traffic counts (24 heads x 664 queries, D 128:
-// 61 us against 72 with one tile). D 256 has LDS for four waves and one tile.
-// Whether the call goes here at all, below 700 items: this kernel takes as long
+// (two workgroups per CU) up to 2.75 per CU; two query tiles per item past
+// that, where there are items enough and K/V traffic counts (24 heads x 664
+// queries, D 128: 61 us against 72 with one tile), and the second tile is not
+// empty (32 x 24 heads, 16 queries over 500 cached keys: 100 us with it, 94
+// without; 24 queries 103 against 168). D 256 has LDS for four waves and one tile.
+// Whether the call goes here at all, below that count: this kernel takes as long
 // as its longest item (T tiles of 16 keys), attn_any_kernel splits the keys of
 // 64-query items until the chip is full. us, s = D / 128, measured over D 32 to
 // 256, 12 to 40 heads, 16 to 2500 queries, 16 to 4000 cached keys:
@@ -318,9 +320,9 @@ F32Plan plan_f32(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_
   F32Plan p{};
   if (D < 32) return p;
   const int64_t items = B * H * ((Lq + 15) / 16);
-  const bool many = D < 256 && items > 700;
+  const bool many = D < 256 && 4 * items > 11 * int64_t(cus);
   p.waves = D < 256 && items <= cus ? 8 : 4;
-  p.qt = many ? 2 : 1;
+  p.qt = many && Lq > 16 ? 2 : 1;
   if (form) {
     p.waves = D < 256 && form == 8 ? 8 : 4;
     p.qt = D < 256 && form == 2 ? 2 : 1;

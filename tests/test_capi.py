@@ -289,3 +289,14 @@ def test_head_dim_256_choice_counts_items_and_rounds(built_lib):
     # A ragged batch: its longest sequence's items bound the launch.
     assert attention_kernel(bf, 4, 200, 200, 16, 256, lens=[100, 100, 100, 8000]) == GENERAL
     assert attention_kernel(bf, 4, 200, 200, 16, 256, lens=[500, 400, 500, 600]) == WIDE
+
+
+def test_fp32_form_leaves_no_empty_query_tile(built_lib):
+    """Two query tiles per item past 2.75 16-query items per CU, one where the second is empty."""
+    f32 = torch.float32
+    assert attention_kernel(f32, 32, 16, 16, 24, 128, 500) == F32_FOUR
+    assert attention_kernel(f32, 64, 1, 1, 16, 64, 2000) == F32_FOUR
+    assert attention_kernel(f32, 32, 17, 17, 24, 128, 500) == F32_PAIR
+    assert attention_kernel(f32, 1, 664, 664, 24, 128) == F32_PAIR
+    assert attention_kernel(f32, 1, 16 * 44, 8, 16, 128) != F32_PAIR  # 704 items on 256 CUs
+    assert attention_kernel(f32, 1, 16 * 44 + 1, 8, 16, 128) == F32_PAIR
