@@ -3697,17 +3697,34 @@ void one_launch(Plan& p, int kernel, int bm, int64_t B, int64_t Lq, int64_t H) {
 //  - More items (4 waves, two workgroups per CU): up to two per CU and T up
 //    to 20 (24 heads, 400 x 640 15.0 -> 13.3; 40 heads, 300 x 768 keys 16.9 ->
 //    15.7, but 200 x 768 14.6 -> 15.3; three items per CU: 1000 x 256 13.4 ->
-//    14.2). Under a causal or block mask of nb > 1 blocks, where the paired
-//    kernel's 256-query items see far more keys than their queries need: up
-//    to 64 (1 - 1/nb) tiles per CU at D 128 (causal 1000 25.2 -> 21.5; 16
-//    heads, causal 1400 26.6 -> 22.5, 2000 36.4 -> 37.8), 96 at D 64 (24
-//    heads, causal 1400 28.6 -> 22.2; 40 heads, 1400 29.8 -> 33.3).
-bool wave_kernel_fits(double items, double tiles, int64_t D, int64_t nb, bool causal, int cus) {
+//    14.2).
+//  - Beyond, under a causal or block mask, whose late queries alone see all new
+//    keys, and not in a ragged batch (four sequences of 99 queries in blocks of
+//    83 over up to 300 cached, 40 heads 18.9 -> 20.9, D 64, eight of 24 heads
+//    15.7 -> 18.5). In place of the dual-stream kernel (at most two items per CU): T up
+//    to 36 (16 heads, 700 over 500 cached 26.9 -> 23.7 in blocks of 83; 24
+//    heads, 332 causal over 700 18.6 -> 18.2, over 1300 22.0 -> 25.8, stays; 8
+//    heads, 1200 causal over 300 20.6 -> 21.1, over 700 22.6 -> 24.6, stays).
+//    In place of the paired kernel, whose 256-query items see far more new keys
+//    than their queries need, but read cached ones, of which every query needs
+//    all, eight times less often: up to 3 items per CU, 4.2 at D 64, and up to
+//    76 (1 - 1/nb) tiles per CU, 128 at D 64, with cached tiles counted twice
+//    (nb blocks; causal: 1). 12 heads, 1500 causal 28.4 -> 23.0; 2 x 24 heads,
+//    300 causal over 500 25.2 -> 20.2; 40 heads, 600 causal 22.6 -> 20.6, over
+//    300 26.9 -> 27.8, stays; 4 x 24 heads, 332 causal 19.7 -> 22.6, 500 in
+//    blocks of 83 27.7 -> 37.2, stay; D 64, 24 heads, 1400 causal 30.4 -> 24.9,
+//    4 x 16 heads, 700 in blocks of 83 26.3 -> 31.8, stays. Of 500 measured
+//    calls the nine wrong ones lose 3 or 4%.
+bool wave_kernel_fits(double items, double tiles, double seen, int64_t D, int64_t nb, bool causal,
+                      bool ragged, bool dual, int cus) {
   const double t = tiles / items;
   if (items <= cus) return t <= (D == 64 || items * 8 >= 3 * cus ? 18 : 14);
   if (items <= 2 * cus && t <= 20) return true;
-  const double masked = causal ? 1.0 : nb > 1 ? 1.0 - 1.0 / double(nb) : 0.0;
-  return tiles / cus <= (D == 64 ? 96 : 64) * masked;
+  if (ragged || (!causal && nb <= 1)) return false;
+  if (dual) return t <= 36;
+  const double masked = causal ? 1.0 : 1.0 - 1.0 / double(nb);
+  return items <= (D == 64 ? 4.2 : 3.0) * cus &&
+         (2 * tiles - items * seen) / cus <= (D == 64 ? 128 : 76) * masked;
 }
 
 // Turn the plan of a call that wave_kernel_fits into one launch of
@@ -3735,7 +3752,9 @@ void use_wave_kernel(Plan& p, int64_t B, int64_t Lq, int64_t Lk, int64_t H, int6
     }
     if (!forced && double(longest) + seen > 20) return;
   }
-  if (!forced && !wave_kernel_fits(double(items), tiles, D, n_blocks, causal, cus)) return;
+  if (!forced && !wave_kernel_fits(double(items), tiles, seen, D, n_blocks, causal,
+                                   p.n_seg > 0, p.kernel == kDual, cus))
+    return;
   const int waves = items <= cus ? 8 : 4;
   if (!grid_fits(items, 64 * waves)) return;
   p.nqw = waves;

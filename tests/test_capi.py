@@ -300,3 +300,23 @@ def test_fp32_form_leaves_no_empty_query_tile(built_lib):
     assert attention_kernel(f32, 1, 664, 664, 24, 128) == F32_PAIR
     assert attention_kernel(f32, 1, 16 * 44, 8, 16, 128) != F32_PAIR  # 704 items on 256 CUs
     assert attention_kernel(f32, 1, 16 * 44 + 1, 8, 16, 128) == F32_PAIR
+
+
+def test_wave_split_choice_counts_cached_keys_and_rounds(built_lib):
+    """A mask makes room for the wave split by the new keys that it hides: not over a long cache,
+    and not in batches whose items pass three per CU (both sides measured)."""
+    bf = torch.bfloat16
+    causal = lambda *a: attention_kernel(bf, *a, causal=True)  # noqa: E731
+    blocks = lambda *a: attention_kernel(bf, *a, n_blocks=-(-a[1] // 83))  # noqa: E731
+    assert causal(1, 332, 332, 24, 128, 700) == WAVE
+    assert causal(1, 332, 332, 24, 128, 1300) == DUAL
+    assert causal(1, 1200, 1200, 8, 128, 700) == DUAL
+    assert causal(1, 600, 600, 40, 128) == WAVE and causal(1, 600, 600, 40, 128, 300) == PAIRED
+    assert causal(2, 300, 300, 24, 128, 500) == WAVE
+    assert causal(4, 332, 332, 24, 128) == PAIRED and causal(6, 500, 500, 16, 128) == PAIRED
+    assert blocks(4, 332, 332, 24, 128) == PAIRED and blocks(2, 332, 332, 24, 128) == WAVE
+    assert blocks(4, 700, 700, 16, 64) == PAIRED and causal(1, 1400, 1400, 24, 64) == WAVE
+    ragged = lambda h, d, lens: attention_kernel(bf, len(lens), 99, 99, h, d, lens=lens,  # noqa: E731
+                                                 n_blocks=2)
+    assert ragged(24, 128, [0, 100, 200, 300]) == WAVE and ragged(40, 128, [0, 100, 200, 300]) == DUAL
+    assert ragged(24, 64, [0, 0, 83, 400, 200, 100, 300, 50]) == DUAL
