@@ -112,11 +112,11 @@ class SelfAttention(nn.Module):
         # 16.7 us); at 5120 it and hipBLASLt are mixed.
         x = out.flatten(2)
         b, seq, dim = x.shape
+        weight, bias = self.o.weight, self.o.bias  # read once: a parametrization computes them
         linear = F.linear
-        if 0 < b * seq <= 128 and dim % 512 == 0 and dim <= 4096 \
-                and _computes_only(self.o.weight, self.o.bias):
+        if 0 < b * seq <= 128 and dim % 512 == 0 and dim <= 4096 and _computes_only(weight, bias):
             try:
-                linear = select("gemm", "linear_chunk", x, self.o.weight, self.o.bias)
+                linear = select("gemm", "linear_chunk", x, weight, bias)
             except LookupError:  # a weight layout the kernel does not take
                 pass
-        return linear(x, self.o.weight, self.o.bias)
+        return linear(x, weight, bias)

@@ -5,6 +5,7 @@ import contextlib
 import pytest
 import torch
 import torch.nn.functional as F
+import torch.nn.utils.parametrize
 from torch.autograd import forward_ad
 
 from dexter_amd.models import attention
@@ -62,3 +63,20 @@ def test_a_weight_subclass_keeps_torchs_linear(monkeypatch):
         m.o.weight = w
 
     assert _project(monkeypatch, 8, 512, edit) == []
+
+
+def test_a_parametrized_weight_is_computed_once(monkeypatch):
+    """A stateful parametrization (spectral norm in training mode) advances one step a call."""
+    class Count(torch.nn.Module):
+        steps = 0
+
+        def forward(self, w):
+            Count.steps += 1
+            return w
+
+    def edit(m):
+        torch.nn.utils.parametrize.register_parametrization(m.o, "weight", Count())
+        Count.steps = 0
+
+    assert _project(monkeypatch, 8, 512, edit) == [("gemm", "linear_chunk")]
+    assert Count.steps == 1
