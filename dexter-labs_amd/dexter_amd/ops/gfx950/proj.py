@@ -122,12 +122,19 @@ def qkv_norm_rope(x, wq, bq, wk, bk, wv, bv, q_weight, k_weight, cos, sin, heads
     return q_out, k_out, v_out
 
 
+# dx_linear_chunk's own limits: features either way, elements from one weight row to the
+# next, and bytes from x's first element to its last.
+_MAX_FEATURES, _MAX_ROW_STEP, _MAX_SPAN = 1 << 20, 1 << 22, 1 << 31
+
+
 def _accepts_linear(x, w, b) -> bool:
     if not (x.is_cuda and x.dtype in MATRIX_DTYPES and x.dim() == 3 and w.dim() == 2):
         return False
     n, c = w.shape
-    return (0 < x.shape[0] * x.shape[1] <= MAX_TOKENS and x.shape[2] == c and c % 512 == 0
-            and n % 16 == 0 and _weight_ok(w, n, c, x.dtype) and w.device == x.device
+    return (0 < x.shape[0] * x.shape[1] <= MAX_TOKENS and x.shape[2] == c
+            and 0 < c <= _MAX_FEATURES and c % 512 == 0 and 0 < n <= _MAX_FEATURES and n % 16 == 0
+            and _weight_ok(w, n, c, x.dtype) and c <= w.stride(0) < _MAX_ROW_STEP
+            and w.device == x.device
             and (b is None or (b.shape == (n,) and b.dtype == x.dtype and b.device == x.device)))
 
 
@@ -135,13 +142,15 @@ def _accepts_linear(x, w, b) -> bool:
           capability=CDNA4, priority=Priority.SPECIALISED, accepts=_accepts_linear)
 def linear_chunk(x, w, b):
     bsz, seq, c = x.shape
-    if not rows_ok(x) or min(x.stride()) < 0:
-        x = x.contiguous()
+    sb, sl = strides(x, 2)
+    if not rows_ok(x) or 2 * ((bsz - 1) * sb + (seq - 1) * sl + c) >= _MAX_SPAN:
+        x = x.clone(memory_format=torch.contiguous_format)  # aligned too, which contiguous() need not be
+        sb, sl = strides(x, 2)
     if b is not None and (b.stride(0) != 1 or b.data_ptr() % 16):
         b = b.clone(memory_format=torch.contiguous_format)
     y = torch.empty((bsz, seq, w.shape[0]), device=x.device, dtype=x.dtype)
     rc = _lib.load().dx_linear_chunk(
-        x.data_ptr(), *strides(x, 2), _lib.dtype_code(x.dtype), w.data_ptr(), w.stride(0),
+        x.data_ptr(), sb, sl, _lib.dtype_code(x.dtype), w.data_ptr(), w.stride(0),
         _lib.ptr(b), y.data_ptr(), bsz, seq, c, w.shape[0], _lib.stream_handle(x.device))
     _lib.check(rc, "linear_chunk")
     return y

@@ -265,13 +265,32 @@ def test_linear_chunk(device, built_lib, b, l, c, n, dtype, bias):
     assert not bad.any(), f"{int(bad.sum())} elements beyond one ulp"
 
 
-def test_output_projection_falls_back(device, built_lib):
+def test_linear_chunk_of_a_view_past_32_bit_offsets(device, built_lib):
+    """Two chunks of a buffer 2 GiB apart."""
+    big = torch.zeros(2, 2**21 + 8, 512, device=device, dtype=DT)
+    x = big[:, 8:16].normal_()
+    w = torch.randn(512, 512, device=device).mul(512 ** -0.5).to(DT)
+    assert torch.equal(ops.linear_chunk(x, w), ops.linear_chunk(x.contiguous(), w))
+
+
+def test_linear_chunk_of_an_unaligned_view(device, built_lib):
+    flat = torch.randn(8 * 512 + 1, device=device).to(DT)
+    x = flat[1:].view(1, 8, 512)
+    w = torch.randn(512, 512, device=device).mul(512 ** -0.5).to(DT)
+    assert torch.equal(ops.linear_chunk(x, w), ops.linear_chunk(x.clone(), w))
+
+
+@pytest.mark.parametrize("layout", ["column-major", "one row"])
+def test_output_projection_falls_back(device, built_lib, layout):
     """A weight layout the chunk GEMM does not take still projects (``F.linear``)."""
     from dexter_amd.models import SelfAttention
     layer = SelfAttention(512, 4, dtype=DT, device=device)
     x = torch.randn(1, 20, 512, device=device).to(DT)
     cos, sin = (t.to(device) for t in rope_table(torch.arange(20), 128))
+    if layout == "one row":
+        layer.o.weight.data[:] = layer.o.weight.data[:1].clone()
     plain = layer(x, cos, sin, None, 0)
-    wt = layer.o.weight.data.t().contiguous()
-    layer.o.weight.data = wt.t()  # column-major
+    weight = layer.o.weight.data
+    layer.o.weight.data = (weight[:1].expand(512, 512) if layout == "one row"
+                           else weight.t().contiguous().t())
     assert_parity_scaled(layer(x, cos, sin, None, 0), plain.float())

@@ -9,6 +9,7 @@ import torch.nn.utils.parametrize
 from torch.autograd import forward_ad
 
 from dexter_amd.models import attention
+from dexter_amd.ops.gfx950 import proj
 
 
 def _project(monkeypatch, tokens, dim, edit=lambda m: None):
@@ -80,3 +81,24 @@ def test_a_parametrized_weight_is_computed_once(monkeypatch):
 
     assert _project(monkeypatch, 8, 512, edit) == [("gemm", "linear_chunk")]
     assert Count.steps == 1
+
+
+class _OnGpu(torch.Tensor):
+    """Passes for a CUDA tensor in the predicate."""
+    is_cuda = True
+
+
+def test_the_kernel_declines_what_its_entry_point_refuses():
+    """Each limit of dx_linear_chunk is the predicate's, so such calls keep torch's linear."""
+    def takes(rows, cols, step=None, tokens=8):
+        step = cols if step is None else step
+        store = torch.empty(max((rows - 1) * step + cols, 1), dtype=torch.bfloat16)
+        w = torch.as_strided(store, (rows, cols), (step, 1)).as_subclass(_OnGpu)
+        x = torch.empty(1, tokens, cols, dtype=torch.bfloat16).as_subclass(_OnGpu)
+        return proj._accepts_linear(x, w, None)
+
+    assert takes(512, 512) and takes(512, 512, 520) and takes(16, 512, 2**22 - 8)
+    assert not takes(512, 512, 0) and not takes(512, 512, 504)  # expanded, overlapping rows
+    assert not takes(16, 512, 2**22)
+    assert not takes(0, 512) and not takes(16, 0)
+    assert not takes(16, 2**20 + 512) and takes(16, 2**20)
