@@ -25,7 +25,7 @@ from torch import nn
 from torch.autograd import forward_ad
 
 from .. import ops
-from ..registry import select
+from ..registry import NoKernelError, select
 from .kv_cache import KVCache
 
 
@@ -117,6 +117,6 @@ class SelfAttention(nn.Module):
         if 0 < b * seq <= 128 and dim % 512 == 0 and dim <= 4096 and _computes_only(weight, bias):
             try:
                 linear = select("gemm", "linear_chunk", x, weight, bias)
-            except LookupError:  # a weight layout the kernel does not take
+            except NoKernelError:  # a weight layout the kernel does not take
                 pass
         return linear(x, weight, bias)

@@ -33,10 +33,15 @@ from typing import Callable, Iterator
 
 from .platform import Capability, PlatformInfo, current_platform
 
-__all__ = ["Priority", "KernelSpec", "register", "select", "select_spec", "candidates",
+__all__ = ["NoKernelError", "Priority", "KernelSpec", "register", "select", "select_spec", "candidates",
            "explain", "registered", "unregister"]
 
 PIN_ENV = "DEXTER_KERNEL"
+
+
+class NoKernelError(LookupError):
+    """No registered implementation takes the call (a pin that cannot be met is a plain
+    ``LookupError``: a caller with another way to compute the call must not hide it)."""
 
 
 class Priority(IntEnum):
@@ -208,8 +213,8 @@ def select_spec(family: str, mode: str, *args, **kwargs) -> KernelSpec:
                 spec.accepts is None or spec.accepts(*args, **kwargs)):
             return spec
     names = [s.name for s in _CATALOGUE.specs(key)]
-    raise LookupError(f"no kernel for {key} on {platform.describe()}. "
-                      f"Registered: {names or 'none'}")
+    raise NoKernelError(f"no kernel for {key} on {platform.describe()}. "
+                        f"Registered: {names or 'none'}")
 
 
 def select(family: str, mode: str, *args, **kwargs) -> Callable:

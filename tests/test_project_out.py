@@ -102,3 +102,15 @@ def test_the_kernel_declines_what_its_entry_point_refuses():
     assert not takes(16, 512, 2**22)
     assert not takes(0, 512) and not takes(16, 0)
     assert not takes(16, 2**20 + 512) and takes(16, 2**20)
+
+
+def test_a_pin_that_cannot_be_met_is_raised(monkeypatch):
+    """As for every other op; without a pin, no kernel for the call means torch's linear."""
+    module = attention.SelfAttention(512, 8, dtype=torch.float32)
+    x = torch.randn(1, 8, 8, 64)
+    with torch.no_grad():
+        plain = module._project_out(x)
+        assert torch.equal(plain, F.linear(x.flatten(2), module.o.weight, module.o.bias))
+        monkeypatch.setenv("DEXTER_KERNEL", "gemm/linear_chunk:mistyped")
+        with pytest.raises(LookupError, match="pinned gemm/linear_chunk:mistyped"):
+            module._project_out(x)
