@@ -23,6 +23,8 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from .. import ops
 from ..registry import NoKernelError, select
@@ -31,10 +33,15 @@ from .kv_cache import KVCache
 
 def _computes_only(*params) -> bool:
     """Whether a torch op on ``params`` would do no more than compute (``forward`` runs
-    without gradients): no autocast, no forward-mode level, no functorch transform and no
-    tensor subclass, all of which a kernel called by address passes by."""
+    without gradients): no autocast, no forward-mode level, no functorch transform, no
+    dispatch or function mode (a default device aside, which leaves a linear alone), no
+    trace and no tensor subclass, all of which a kernel called by address passes by."""
     return (not torch.is_autocast_enabled("cuda") and forward_ad._current_level < 0
             and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0
+            and (torch._C._len_torch_function_stack() == 0
+                 or all(type(m) is DeviceContext for m in _get_current_function_mode_stack()))
+            and torch._C._get_tracing_state() is None
             and all(p is None or type(p) in (nn.Parameter, torch.Tensor) for p in params))
 
 

@@ -7,6 +7,8 @@ import torch
 import torch.nn.functional as F
 import torch.nn.utils.parametrize
 from torch.autograd import forward_ad
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from dexter_amd.models import attention
 from dexter_amd.ops.gfx950 import proj
@@ -52,6 +54,42 @@ def test_torch_transforms_keep_torchs_linear(monkeypatch, inside):
         if inside == "autocast" and not torch.is_autocast_enabled("cuda"):
             pytest.skip("torch turns CUDA autocast off without a device")
         assert _project(monkeypatch, 8, 512) == []
+
+
+@pytest.mark.parametrize("mode", ["dispatch", "function"])
+def test_a_torch_mode_sees_the_projection(monkeypatch, mode):
+    seen = []
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    module = attention.SelfAttention(512, 8, dtype=torch.float32)
+    calls = []
+    monkeypatch.setattr(attention, "select", lambda *args: calls.append(args) or F.linear)
+    with torch.no_grad(), Dispatch() if mode == "dispatch" else Function():
+        module._project_out(torch.randn(1, 8, 8, 64))
+    assert not calls
+    assert any(f is F.linear or "mm" in str(f) or "linear" in str(f) for f in seen)
+
+
+def test_a_default_device_keeps_the_kernel(monkeypatch):
+    with torch.device("cpu"):
+        assert _project(monkeypatch, 8, 512) == [("gemm", "linear_chunk")]
+
+
+def test_a_trace_records_torchs_linear(monkeypatch):
+    module = attention.SelfAttention(512, 8, dtype=torch.float32).requires_grad_(False)
+    monkeypatch.setattr(attention, "select", lambda *args: pytest.fail("kernel under a trace"))
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda x: module._project_out(x), torch.randn(1, 8, 8, 64))
+    assert "aten::linear" in str(traced.graph)
 
 
 def test_a_weight_subclass_keeps_torchs_linear(monkeypatch):
