@@ -88,7 +88,8 @@ def test_a_trace_records_torchs_linear(monkeypatch):
     module = attention.SelfAttention(512, 8, dtype=torch.float32).requires_grad_(False)
     monkeypatch.setattr(attention, "select", lambda *args: pytest.fail("kernel under a trace"))
     with torch.no_grad():
-        traced = torch.jit.trace(lambda x: module._project_out(x), torch.randn(1, 8, 8, 64))
+        traced = torch.jit.trace(lambda x: module._project_out(x), torch.randn(1, 8, 8, 64),
+                                 check_trace=False)
     assert "aten::linear" in str(traced.graph)
 
 
