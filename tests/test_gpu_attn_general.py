@@ -291,6 +291,19 @@ def _wide_heads_scales_cursor_ragged(device, scale):
         assert_parity(rag[i:i + 1], ref, what=f"seq {i}")
 
 
+def test_wide_heads_future_keys_never_reach_the_result(device, built_lib):
+    """Inf and NaN in keys that a work item's 128 queries cannot see leave its rows bit for bit."""
+    q, k, v = (torch.randn(1, 400, 16, 256, device=device).bfloat16() for _ in range(3))
+    bb = torch.tensor([0, 100, 256], device=device)
+    k2, v2 = k.clone(), v.clone()
+    k2[:, 256:], v2[:, 256:] = float("inf"), float("nan")
+    with _lib.tuning(_lib.TUNE_ATTN_KERNEL, WIDE):
+        base = ops.blockwise_causal_attention(q, k, v, block_boundaries=bb)
+        got = ops.blockwise_causal_attention(q, k2, v2, block_boundaries=bb)
+    assert torch.equal(got[:, :256], base[:, :256])
+    assert torch.isnan(got[:, 256:]).all()
+
+
 # The fp32 kernel that deals 16-key tiles to a workgroup's waves (attn_f32.hip) at the
 # edges of its tiles and in each of its forms, forced (eight waves; four waves; four waves
 # and two query tiles per item; head dim 256 has four waves and one tile). Bar: fp32 sums in another
