@@ -61,7 +61,6 @@
 
 #include <algorithm>
 #include <mutex>
-#include <set>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -3346,23 +3345,6 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(AttnArgs 
 // ---------------------------------------------------------------------------
 // Host side: launch planning shared by the workspace query and the launch.
 // ---------------------------------------------------------------------------
-int device_cus() {
-  static std::mutex mu;
-  static std::vector<int> cache;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  std::lock_guard<std::mutex> lk(mu);
-  if (int(cache.size()) <= dev) cache.resize(dev + 1, 0);
-  if (cache[dev] == 0) {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus <= 0)
-      cus = 256;
-    cache[dev] = cus;
-  }
-  return cache[dev];
-}
-
 // Attention kernels a plan can pick (the DX_TUNE_ATTN_KERNEL values, and what
 // dx_attention_kernel reports): those of this file, then the general ones.
 enum AttnKernel {

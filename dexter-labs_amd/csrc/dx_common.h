@@ -125,6 +125,8 @@ namespace dx {
 void set_error(const char* fmt, ...);
 // Current value of a dx_set_tuning override (0: the library's own choice).
 int tuning(int key);
+// Compute units of the current device (256 where there is none).
+int device_cus();
 // Opt a kernel into `bytes` of dynamic LDS (beyond the 64 KB default window;
 // gfx950 allows 160 KB per workgroup) on the current device.
 hipError_t opt_in_lds(const void* fn, int bytes);

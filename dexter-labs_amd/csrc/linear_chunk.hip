@@ -258,10 +258,10 @@ hipError_t launch_nt(const LinearArgs& a, int nm, int blocks, hipStream_t st) {
 // (1, 2 or 4) that leave at most one workgroup per CU.
 template <typename T>
 hipError_t launch_t(LinearArgs a, hipStream_t st) {
-  const int tiles = a.N / 16;
+  const int tiles = a.N / 16, cus = device_cus();
   a.groups = a.M > 64 ? 2 : 1;
   int nt = 1;
-  while (nt < 4 && (tiles + nt - 1) / nt * a.groups > 256) nt *= 2;
+  while (nt < 4 && (tiles + nt - 1) / nt * a.groups > cus) nt *= 2;
   int nm = std::max(2, (a.M + 16 * a.groups - 1) / (16 * a.groups));
   if (nt == 1 && nm == 3) nm = 4;  // one of the two counts has to halve
   const int blocks = ((tiles + nt - 1) / nt + 7) / 8 * 8 * a.groups;
