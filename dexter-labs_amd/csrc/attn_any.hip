@@ -306,7 +306,7 @@ __global__ __launch_bounds__(kAnyThreads) void attn_any_kernel(AttnArgs a) {
     for (int u = 0; u < DG; ++u) E::store4(orow + (16 * u + 4 * g) * es, o[u] * inv);
     return;
   }
-  // Partial of this split: row 16 wave + c of item blockIdx.x.
+  // Partial of this split: row 16 wave + c of the item's partial.
   const int64_t prow = it.partial * kAnyRows + 16 * wave + c;
   float* po = reinterpret_cast<float*>(a.ws_o) + prow * D + 4 * g;
 #pragma unroll

@@ -24,10 +24,14 @@
 //    add them in wave order through LDS.
 //
 // 332 queries over 996 + 332 keys in 83-token blocks, 24 heads x 128: 136 -> 62
-// us (79 TFLOP/s of 157 in fp32 MFMA; two rounds of items, ~8 us of each are
-// its start and merge), and the error against 64 bits 7.4e-7 -> 3.7e-7 (shorter
-// chains). Measured and left out, with cold K/V: tiles (V alone) by registers instead
-// of DMA 81 (78) against 74 us, the query rows through LDS 74.
+// us (79 TFLOP/s of 157 in fp32 MFMA), and the error against 64 bits 7.4e-7 ->
+// 3.7e-7 (shorter chains). Its 504 items run at once, two to a CU, one wave of
+// each on a SIMD. Counters: the MFMA units are busy 46% of the launch; a wave
+// waits 27% of its time for its tiles and 51% to issue, behind its own and the
+// other wave's dependent chains; a SIMD holds 1.56 of its two waves on average
+// (items see 69 to 84 tiles). Measured and left out, with cold K/V: tiles (V
+// alone) by registers instead of DMA 81 (78) against 74 us, the query rows
+// through LDS 74.
 #include "attn_tile.h"
 
 #include <algorithm>
