@@ -92,29 +92,6 @@ template <typename T> struct Elem16 {
 template <> struct Elem<bf16_t> : Elem16<bf16_t> {};
 template <> struct Elem<f16_t> : Elem16<f16_t> {};
 
-// Max and sum over the four lanes of a query (lanes c, c + 16, c + 32,
-// c + 48): the gfx950 row swaps, VALU exchanges with no LDS round trip.
-__device__ __forceinline__ float quad_max(float x) {
-  const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x),
-                                                    false, false);
-  x = fmaxf(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
-  const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x),
-                                                    false, false);
-  return fmaxf(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
-}
-__device__ __forceinline__ float quad_sum(float x) {
-  const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x),
-                                                    false, false);
-  x = __uint_as_float(r16[0]) + __uint_as_float(r16[1]);
-  const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x),
-                                                    false, false);
-  return __uint_as_float(r32[0]) + __uint_as_float(r32[1]);
-}
-
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
 template <int D> struct AnyLds {
   static constexpr int RS = D + 4;                      // row stride in floats
   static constexpr int tile = kAnyKeys * RS;            // floats per K or V tile
@@ -332,28 +309,6 @@ __global__ __launch_bounds__(kAnyThreads) void attn_any_kernel(AttnArgs a) {
 //    lanes 4 e + i / 4, e = 0..3; lane 4 e + t addresses row 4 g + e, or
 //    16 + 4 g + e, at columns 16 u + 4 t .. + 3). l sums the rounded
 //    probabilities, the values the product uses.
-template <typename T> struct Mfma16;
-template <> struct Mfma16<bf16_t> {
-  static __device__ __forceinline__ f32x4 run(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
-};
-template <> struct Mfma16<f16_t> {
-  static __device__ __forceinline__ f32x4 run(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-};
-
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ u32x2 lds_tr16(const uint16_t* p) {
-  typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-  const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (lds_v4i16*)((__attribute__((address_space(3))) uint16_t*)(p)));
-  return __builtin_bit_cast(u32x2, r);
-}
-
 template <int D> struct Any16Lds {
   static constexpr int RS = D + 8;             // row stride in 16-bit elements
   static constexpr int tile = kAnyKeys * RS;   // elements per K or V tile
@@ -518,8 +473,8 @@ __global__ __launch_bounds__(kAnyThreads) void attn_any16_kernel(AttnArgs a) {
     for (int u = 0; u < DG; ++u) o[u] *= corr;
 #pragma unroll
     for (int u = 0; u < DG; ++u) {
-      const u32x2 lo = lds_tr16(vt + tr_lo + 16 * u);
-      const u32x2 hi = lds_tr16(vt + tr_hi + 16 * u);
+      const u32x2 lo = lds_read_tr16(vt + tr_lo + 16 * u);
+      const u32x2 hi = lds_read_tr16(vt + tr_hi + 16 * u);
       o[u] = Mfma16<T>::run(u32x4{lo[0], lo[1], hi[0], hi[1]}, pb, o[u]);
     }
     if (t + 1 < t_end) store_tile(stage ^ 1);

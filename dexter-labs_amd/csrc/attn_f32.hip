@@ -55,20 +55,6 @@ template <int D, int QT, int NW> struct F32Shape {
   static __device__ __forceinline__ int swz(int r) { return CR >= 16 ? r & 15 : (r >> 1) & 7; }
 };
 
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-// Max (sum) over the four lane groups holding one query's keys.
-__device__ __forceinline__ float groups_max(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
-                                                  false);
-  return xor32_max(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
-}
-__device__ __forceinline__ float groups_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
-                                                  false);
-  return xor32_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
-}
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t f32_rsrc(const float* base, int rows,
                                                           int row_bytes, int D) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0,
@@ -203,7 +189,7 @@ __global__ __launch_bounds__(64 * NW, 1) void attn_f32_kernel(AttnArgs a) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) s[r] = r < lim ? s[r] : kNegInf;
       }
-      const float mn = fmaxf(m[t], groups_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
+      const float mn = fmaxf(m[t], quad_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
       const float ref = mn == kNegInf ? 0.f : mn;  // nothing visible yet: every p is 0
       if (__any(mn > m[t])) {
         const float corr = fast_exp2(m[t] - ref);
@@ -239,7 +225,7 @@ __global__ __launch_bounds__(64 * NW, 1) void attn_f32_kernel(AttnArgs a) {
   f32x2* const ml = reinterpret_cast<f32x2*>(smem + S::ml);
 #pragma unroll
   for (int t = 0; t < QT; ++t) {
-    l[t] = groups_sum(l[t]);
+    l[t] = quad_sum(l[t]);
     if (g == 0) ml[wid * S::rows + 16 * t + c] = f32x2{m[t], l[t]};
   }
   __syncthreads();  // every wave's tile reads and DMA pieces are done too

@@ -1,6 +1,6 @@
-// Tile-level pieces shared by the attention kernels' sources: 16-bit MFMA,
-// bounded buffer descriptors, LDS reads, lane exchanges, and the work items of
-// the general kernels.
+// Tile-level pieces shared by the kernels' sources: MFMA forms, bounded buffer
+// descriptors, LDS reads, lane exchanges, and the work items of the general
+// attention kernels.
 #pragma once
 
 #include "attn_common.h"
@@ -8,6 +8,7 @@
 namespace dx {
 namespace {
 
+// 32 x 32 x 16 products, and packing to their 16-bit operands.
 template <typename T> struct Mfma;
 template <> struct Mfma<bf16_t> {
   static __device__ __forceinline__ f32x16 run(u32x4 a, u32x4 b, f32x16 c) {
@@ -43,6 +44,24 @@ template <> struct Mfma<f16_t> {
                                   __builtin_bit_cast(f16x2, 0x3c003c00u), acc, false);
   }
 };
+
+// 16 x 16 x 32 (16-bit) and 16 x 16 x 4 (fp32) products.
+template <typename T> struct Mfma16;
+template <> struct Mfma16<bf16_t> {
+  static __device__ __forceinline__ f32x4 run(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+};
+template <> struct Mfma16<f16_t> {
+  static __device__ __forceinline__ f32x4 run(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+};
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -92,6 +111,19 @@ __device__ __forceinline__ float xor32_sum(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
                                                   false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Max and sum over the four lanes of a query of the 16 x 16 products (lanes c,
+// c + 16, c + 32, c + 48): the row swaps, again VALU exchanges.
+__device__ __forceinline__ float quad_max(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  return xor32_max(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
+__device__ __forceinline__ float quad_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  return xor32_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
 }
 
 // Key of register r of half kt: row 32 kt + 8 (r / 4) + 4 g + r % 4 of the

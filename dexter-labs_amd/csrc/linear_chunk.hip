@@ -30,7 +30,7 @@
 // 1536 x 1536: 83 tokens 6.6 (7.4), 24 5.4 (7.2). At 5120 x 5120 the two are
 // mixed (64 tokens 22.2 against 22.5, 83 24.6 against 22.6), so the model
 // takes this kernel up to 4096 features.
-#include "dx_common.h"
+#include "attn_tile.h"
 
 #include <algorithm>
 
@@ -51,26 +51,6 @@ constexpr int kSteps = 4;                  // MFMA steps (of 32) per chunk
 constexpr int kChunkK = 32 * kSteps;       // reduction elements per chunk
 constexpr int kRowB = 2 * kChunkK;         // bytes per staged row
 constexpr int kPieceRows = 1024 / kRowB;   // rows per DMA piece
-constexpr int kWord3 = 0x00020000;         // gfx9-family raw buffer descriptor word 3
-
-template <typename T> struct Mfma16x16;
-template <> struct Mfma16x16<bf16_t> {
-  static __device__ __forceinline__ f32x4 run(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
-};
-template <> struct Mfma16x16<f16_t> {
-  static __device__ __forceinline__ f32x4 run(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-};
-
-typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-__device__ __forceinline__ u32x4 lds_read16(uint32_t at) {
-  return *reinterpret_cast<const lds_u32x4*>(at);
-}
 
 template <int NT, int NM> struct LinearLds {
   static constexpr int rows = 16 * (NT + NM);
@@ -93,7 +73,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void linear_chunk_kernel(LinearArgs
   constexpr int kWPieces = NT * 16 / kPieceRows;
   constexpr int kMaxSlots = (L::rows / kPieceRows + kWaves - 1) / kWaves;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const uint32_t lds = uint32_t(uintptr_t((__attribute__((address_space(3))) char*)smem));
+  const uint32_t lds = lds_addr(smem);
 
   const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
   const int lane = int(threadIdx.x) & 63, n = lane & 15, g = lane >> 4;
@@ -124,11 +104,11 @@ __global__ __launch_bounds__(64 * kWaves, 1) void linear_chunk_kernel(LinearArgs
       const int t = min(t0 + p / 4, tiles - 1);
       rs[i] = __builtin_amdgcn_make_buffer_rsrc(
           const_cast<uint16_t*>(a.w + int64_t(t) * 16 * a.w_row), (short)0,
-          int((15 * a.w_row + a.C) * 2), kWord3);
+          int((15 * a.w_row + a.C) * 2), kBufWord3);
       off[i] = uint32_t(row & 15) * uint32_t(a.w_row) * 2 + col;
     } else {
       rs[i] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.x), (short)0,
-                                                int(x_bytes), kWord3);
+                                                int(x_bytes), kBufWord3);
       const uint32_t m = uint32_t(m0 + min(row - 16 * NT, rows - 1)), b = m / uint32_t(a.L);
       off[i] = uint32_t((int64_t(b) * a.x_sb + int64_t(m - b * uint32_t(a.L)) * a.x_sl) * 2) + col;
     }
@@ -182,17 +162,17 @@ __global__ __launch_bounds__(64 * kWaves, 1) void linear_chunk_kernel(LinearArgs
     if (c + NS - 1 < chunks) send(c + NS - 1, st == 0 ? NS - 1 : st - 1);
     const uint32_t base = at + uint32_t(st) * L::stage;
 #pragma unroll
-    for (int j = 0; j < NF; ++j) w[r][j] = lds_read16(base + uint32_t(jh + j) * 16 * kRowB);
+    for (int j = 0; j < NF; ++j) w[r][j] = lds_read_b128_at(base + uint32_t(jh + j) * 16 * kRowB);
 #pragma unroll
     for (int i = 0; i < NH; ++i)
-      x[r][i] = lds_read16(base + uint32_t(NT + ih + i) * 16 * kRowB);
+      x[r][i] = lds_read_b128_at(base + uint32_t(NT + ih + i) * 16 * kRowB);
     st = st + 1 == NS ? 0 : st + 1;
   };
   auto multiply = [&](int r) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < NH; ++i)
 #pragma unroll
-      for (int j = 0; j < NF; ++j) acc[j][i] = Mfma16x16<T>::run(w[r][j], x[r][i], acc[j][i]);
+      for (int j = 0; j < NF; ++j) acc[j][i] = Mfma16<T>::run(w[r][j], x[r][i], acc[j][i]);
   };
   fetch(0, 0);  // chunks: a multiple of 4
   for (int c = 1; c < chunks - 1; c += 2) {
