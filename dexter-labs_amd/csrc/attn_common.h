@@ -229,11 +229,12 @@ hipError_t launch_wide(AttnArgs a, int dtype, hipStream_t st);
 
 // fp32 inputs at head dims 32 to 256, keys dealt to a workgroup's waves
 // (attn_f32.hip): the form of the launch, and whether it is the faster one.
-// form: 0 the plan's own; else forced: 8 or 4 waves with one query tile, or 2
+// splits: as for wide_fits. form: 0 the plan's own; else forced: 8 or 4 waves with one query tile, or 2
 // for four waves with two (as far as the head dim has that form).
 struct F32Plan { bool fits; int waves, qt; };
 F32Plan plan_f32(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_t cache_len,
-                 const int64_t* cache_lens, int64_t n_blocks, bool causal, int cus, int form);
+                 const int64_t* cache_lens, int64_t n_blocks, bool causal, int splits, int cus,
+                 int form);
 hipError_t launch_f32(AttnArgs a, int D, const F32Plan& p, hipStream_t st);
 
 }  // namespace dx

@@ -35,6 +35,7 @@
 #include "attn_tile.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace dx {
 namespace {
@@ -290,55 +291,90 @@ hipError_t launch_d(const AttnArgs& a, const F32Plan& p, hipStream_t st) {
 }  // namespace
 
 // Form by the 16-query items I: eight waves up to one item per CU; four waves
-// (two workgroups per CU) up to 2.75 per CU; two query tiles per item past
-// that, where there are items enough and K/V traffic counts (24 heads x 664
-// queries, D 128: 61 us against 72 with one tile), and the second tile is not
-// empty (32 x 24 heads, 16 queries over 500 cached keys: 100 us with it, 94
-// without; 24 queries 103 against 168). D 256 has LDS for four waves and one tile.
-// Whether the call goes here at all, below that count: this kernel takes as long
-// as its longest item (T tiles of 16 keys), attn_any_kernel splits the keys of
-// 64-query items until the chip is full. us, s = D / 128, measured over D 32 to
-// 256, 12 to 40 heads, 16 to 2500 queries, 16 to 4000 cached keys:
-//   8 waves 7 + 0.4 s T; 4 waves 8 + 0.75 s T (D 256: per round of items over
-//   the CUs, 8 + 0.78 T); attn_any_kernel 13 + 9 s + 0.0057 s per 64-query item
-//   and tile.
-// D 128, that kernel -> this one: 83 x 24 heads over 512 keys 36.2 -> 20.5,
-// over 1083 40.5 -> 34.5, over 4083 95 -> 96 (stays); 664 x 24 heads 116 -> 61,
-// causal 75 -> 48; 2500 x 12 heads 414 -> 358. D 16 is not measured and stays.
+// up to 2.75 per CU; two query tiles per item past that, where there are items
+// enough and K/V traffic counts (24 heads x 664 queries, D 128: 61 us against 72
+// with one tile), and the second tile is not empty (32 x 24 heads, 16 queries
+// over 500 cached keys: 100 us with it, 94 without; 24 queries 103 against
+// 168). D 256 has LDS for four waves and one tile.
+//
+// Whether the call goes here at all: modelled times (us, s = D / 128) of the
+// form and of attn_any_kernel. A CU's n items take the longest of: one wave's
+// own chain of tiles, the matrix units' time for the tiles of all n, and the
+// call's K/V from HBM at 5.8 TB/s, once, or once per round of resident items
+// where it exceeds the 256 MB cache (a head's query tiles run in different
+// rounds); then a fixed time, and one per item:
+//                      fixed     chain         all          item
+//   eight waves        8.8       3.3 s         -            -
+//   four               5.9       0.6 + 1.3 s   1.45 s       0.15 + 1.8 s
+//   four, two tiles    5.0       0.4 + 2.1 s   0.05 + 2.1 s 1.6 + 3.3 s
+//   attn_any_kernel    4.9 (+ 7.1 s if split)  0.5 + 2.6 s  2.65 s  3.2
+// by 16-key tiles dealt to an item's waves, or (attn_any_kernel, 64 queries an
+// item, 32-key tiles) to its key splits. K/V counts a head's per query head.
+// Fitted to 950 calls (1 to 64 sequences, 1 to 8000 queries, 16 to 4500 keys, D
+// 32 to 256): nine of them run more than 3% slower than on the general kernel,
+// and 22 would be that much faster here. Cold, us, that kernel -> this one, D
+// 128: 332 x 24 heads over 996 in blocks of 83 136 -> 67; 400 x 24 over 500 96
+// -> 77; 83 x 24 over 512 keys 36 -> 21; 2500 x 12 heads 416 -> 360. Stays: one
+// query, 24 heads over 1000 23.5 (30.5 here); 4 x 24 heads, 300 onto 64 keys
+// 23.6 (28.5); 32 x 16 heads, 64 over 1000 197 (220); 24 heads, 2000 onto 128
+// keys 47 (53); 64 heads, 4000 onto 16 83 (145); D 256, 32 x 16 heads, 40 over
+// 1000 423 (561). D 16 is not measured and stays.
 F32Plan plan_f32(int64_t B, int64_t Lq, int64_t Lk, int64_t H, int64_t D, int64_t cache_len,
-                 const int64_t* cache_lens, int64_t n_blocks, bool causal, int cus, int form) {
+                 const int64_t* cache_lens, int64_t n_blocks, bool causal, int splits, int cus,
+                 int form) {
   F32Plan p{};
   if (D < 32) return p;
-  const int64_t items = B * H * ((Lq + 15) / 16);
-  const bool many = D < 256 && 4 * items > 11 * int64_t(cus);
+  auto cdiv = [](int64_t x, int64_t y) { return (x + y - 1) / y; };
+  const int64_t items = B * H * cdiv(Lq, 16);
   p.waves = D < 256 && items <= cus ? 8 : 4;
-  p.qt = many && Lq > 16 ? 2 : 1;
+  p.qt = D < 256 && 4 * items > 11 * int64_t(cus) && Lq > 16 ? 2 : 1;
   if (form) {
     p.waves = D < 256 && form == 8 ? 8 : 4;
     p.qt = D < 256 && form == 2 ? 2 : 1;
   }
-  const int64_t blocks = B * H * ((Lq + 16 * p.qt - 1) / (16 * p.qt));
+  const int64_t blocks = B * H * cdiv(Lq, 16 * p.qt);
   if (!grid_fits(blocks, 64 * p.waves)) return p;
-  p.fits = many || form;
-  if (p.fits) return p;
-  auto tiles = [](int64_t keys) { return double((keys + kKeys - 1) / kKeys); };
-  double seen = tiles(Lk);  // mean new-key tiles of an item
-  if (causal) seen = (seen + 1) / 2;
-  else if (n_blocks > 1) seen *= double(n_blocks + 1) / double(2 * n_blocks);
-  const double per_seq = double(H * ((Lq + 63) / 64));
-  double longest = 0, all = 0;
-  for (int64_t i = 0; i < B; ++i) {
-    const double c = tiles(cache_lens ? cache_lens[i] : cache_len);
-    longest = std::max(longest, c);
-    all += per_seq * (c + seen);
+  p.fits = form != 0;
+  if (form) return p;
+
+  // 16- and 32-key tiles of the mean item and of the longest one.
+  double mean[2], longest[2];
+  for (int k = 0; k < 2; ++k) {
+    const int64_t keys = 16 << k;
+    double seen = double(cdiv(Lk, keys));
+    longest[k] = mean[k] = 0;
+    for (int64_t i = 0; i < (cache_lens ? B : 1); ++i) {
+      const double c = double(cdiv(cache_lens ? cache_lens[i] : cache_len, keys));
+      longest[k] = std::max(longest[k], c);
+      mean[k] += c / double(cache_lens ? B : 1);
+    }
+    longest[k] += seen;
+    if (causal) seen = (seen + 1) / 2;
+    else if (n_blocks > 1) seen *= double(n_blocks + 1) / double(2 * n_blocks);
+    mean[k] += seen;
   }
-  longest += tiles(Lk);
-  const double s = double(D) / 128;
-  const double here = D == 256 ? double((items + cus - 1) / cus) * (8 + 0.78 * longest)
-                      : p.waves == 8 ? 7 + 0.4 * s * longest
-                                     : double((items + 2 * cus - 1) / (2 * cus)) *
-                                           (8 + 0.75 * s * longest);
-  p.fits = here <= 13 + 9 * s + 0.0057 * s * all;
+  const double s = double(D) / 128, kv_bytes = double(B * H) * mean[0] * 16 * double(D) * 8;
+  // Resident workgroups per CU: by LDS, or the two-tile form's registers.
+  const double by_lds = 256.0 / double(D), by_regs = 1 + 128.0 / double(D);
+  auto time = [&](int k, double workgroups, double per_cu, int64_t q_tiles, double parts,
+                  double fixed, double chain, double all, double item) {
+    const double n = std::ceil(workgroups / cus), rounds = std::ceil(workgroups / (per_cu * cus));
+    const double reads = kv_bytes > 256e6 ? std::min(double(q_tiles), rounds) : 1;
+    const double tiles = std::max(std::ceil(longest[k] / parts) * chain,
+                                  n * std::ceil(mean[k] / parts) * all);
+    return fixed + std::max(tiles, reads * kv_bytes / 5.8e6) + n * item;
+  };
+  const int64_t q_tiles = cdiv(Lq, 16 * p.qt), q_tiles64 = cdiv(Lq, 64);
+  const double here =
+      p.waves == 8 ? time(0, double(blocks), by_lds, q_tiles, 8, 8.8, 3.3 * s, 0, 0)
+      : p.qt == 1  ? time(0, double(blocks), by_lds, q_tiles, 4, 5.9, 0.6 + 1.3 * s, 1.45 * s,
+                          0.15 + 1.8 * s)
+                   : time(0, double(blocks), by_regs, q_tiles, 4, 5.0, 0.4 + 2.1 * s,
+                          0.05 + 2.1 * s, 1.6 + 3.3 * s);
+  const double there =
+      time(1, double(B * H * q_tiles64 * splits), by_lds, q_tiles64, splits,
+           4.9 + (splits > 1 ? 7.1 * s : 0), 0.5 + 2.6 * s, 2.65 * s, 3.2);
+  p.fits = here <= there;
   return p;
 }
 

@@ -3800,7 +3800,7 @@ int route_call(const CallShape& c, Route& r) {
   if (c.dtype == DX_F32) {
     const int form = forced == kF32Eight ? 8 : forced == kF32Four ? 4 : forced == kF32Pair ? 2 : 0;
     r.pf = plan_f32(c.B, c.Lq, c.Lk, c.H, c.D, c.cache_len, c.cache_lens, c.n_blocks, c.causal,
-                    cus, form);
+                    r.pa.splits, cus, form);
     if (r.pf.fits)
       r.kernel = r.pf.waves == 8 ? kF32Eight : r.pf.qt == 2 ? kF32Pair : kF32Four;
   } else if (c.D == 256 && q_rows_fit(std::min<int64_t>(c.Lq, kWideQ), c.q_sl, c.D) &&

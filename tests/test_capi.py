@@ -263,8 +263,8 @@ def test_grids_past_the_launch_limit(built_lib):
     """A launch holds less than 2^32 threads: calls whose finer work items pass that stay on the
     general kernel, which has fewer of them."""
     f32, bf = torch.float32, torch.bfloat16
-    assert attention_kernel(f32, 1, 2**23 - 32, 64, 64, 32) == F32_PAIR
-    assert attention_kernel(f32, 1, 2**23, 64, 64, 32) == GENERAL
+    assert attention_kernel(f32, 1, 2**23 - 32, 2048, 64, 32) == F32_PAIR
+    assert attention_kernel(f32, 1, 2**23, 2048, 64, 32) == GENERAL
     with _lib.tuning(_lib.TUNE_ATTN_KERNEL, WIDE):
         assert attention_kernel(bf, 1 << 10, 1, 32, (1 << 13) - 1, 256) == WIDE
         assert attention_kernel(bf, 1 << 10, 1, 32, 1 << 13, 256) == GENERAL
@@ -298,8 +298,24 @@ def test_fp32_form_leaves_no_empty_query_tile(built_lib):
     assert attention_kernel(f32, 64, 1, 1, 16, 64, 2000) == F32_FOUR
     assert attention_kernel(f32, 32, 17, 17, 24, 128, 500) == F32_PAIR
     assert attention_kernel(f32, 1, 664, 664, 24, 128) == F32_PAIR
-    assert attention_kernel(f32, 1, 16 * 44, 8, 16, 128) != F32_PAIR  # 704 items on 256 CUs
-    assert attention_kernel(f32, 1, 16 * 44 + 1, 8, 16, 128) == F32_PAIR
+    assert attention_kernel(f32, 1, 16 * 44, 500, 16, 128) == F32_FOUR  # 704 items on 256 CUs
+    assert attention_kernel(f32, 1, 16 * 44 + 1, 500, 16, 128) == F32_PAIR
+
+
+def test_fp32_choice_counts_items_and_rounds(built_lib):
+    """Short key ranges, and batches whose 16-query items take more rounds, stay on the general
+    kernel; the others go to the fp32 wave split (both measured)."""
+    f32 = torch.float32
+    for b, lq, lk, h, d, cache in [(4, 300, 64, 24, 128, 0), (1, 4000, 16, 64, 128, 0),
+                                   (32, 64, 64, 16, 128, 1000), (32, 40, 40, 16, 64, 4000),
+                                   (32, 40, 40, 16, 256, 1000), (1, 1, 1, 24, 64, 1000),
+                                   (2, 1, 1, 24, 32, 4000), (1, 83, 83, 24, 128, 4000)]:
+        assert attention_kernel(f32, b, lq, lk, h, d, cache) == GENERAL, (b, lq, lk, h, d, cache)
+    for b, lq, lk, h, d, cache in [(1, 83, 512, 24, 128, 0), (1, 332, 332, 24, 128, 996),
+                                   (1, 400, 400, 24, 128, 500), (1, 2500, 2500, 12, 128, 0),
+                                   (32, 16, 16, 24, 128, 2000), (1, 200, 200, 40, 64, 4000),
+                                   (17, 40, 40, 16, 32, 1000), (2, 16, 16, 24, 256, 1000)]:
+        assert attention_kernel(f32, b, lq, lk, h, d, cache) > GENERAL, (b, lq, lk, h, d, cache)
 
 
 def test_wave_split_choice_counts_cached_keys_and_rounds(built_lib):
