@@ -60,7 +60,8 @@ struct AttnArgs {
   uint32_t fast_ticks;
   // Dual-stream kernel, split groups merged in the launch: spread the merge
   // over the group's splits (spread_split_group) instead of leaving it to
-  // the last one to arrive (arrive_split_group).
+  // the last one to arrive (arrive_split_group). General kernels: a head's key
+  // splits on consecutive workgroups, and so on every XCD (any_item).
   int spread;
   int seg_b[kMaxSeg], seg_splits[kMaxSeg], seg_cache[kMaxSeg];
   int seg_base[kMaxSeg + 1], comb_base[kMaxSeg + 1];

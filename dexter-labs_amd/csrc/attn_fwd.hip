@@ -4058,6 +4058,7 @@ int attention_entry(const void* q, int64_t q_sb, int64_t q_sl, int64_t q_sh, con
     a.causal = causal != 0;
     a.n_qtiles = pa.n_qtiles;
     a.n_splits = pa.splits;
+    a.spread = r.kernel == kGeneral && pa.n_qtiles == 1 && H == Hkv && pa.items <= device_cus();
     // Signed: the kernel masks by selection after the product, so a negative
     // or zero scale needs no special form.
     a.scale_log2 = softmax_scale * 1.4426950408889634f;

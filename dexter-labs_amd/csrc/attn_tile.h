@@ -148,6 +148,11 @@ __device__ __forceinline__ int any_cache_len(const AttnArgs& a, int b) {
 // call, before (split fastest, then query tiles in order) -> now: D 256 causal
 // 4000, 16 over 4 heads 467 -> 315; D 32 causal 4096 155 -> 91; D 256, 40 heads
 // x 1500 in blocks of 200 198 -> 153; 2048 unmasked 166 -> 159.
+// Where one work item reads each key (one query tile, a K/V head per query
+// head) and all run at once (at most one per CU), an L2 has nothing to share:
+// there a.spread keeps the splits of a head on consecutive workgroups. D 256, 64
+// queries, 24 heads over 500 cached 21.9 us without it, 19.9 with it, 40 heads
+// over 300 21.8 and 19.1; past one item per CU 24 heads over 1245 26.9 and 27.7.
 struct AnyItem {
   int b, h, qt, split;
   int64_t partial;
@@ -155,7 +160,10 @@ struct AnyItem {
 __device__ __forceinline__ AnyItem any_item(const AttnArgs& a, int i) {
   const uint32_t G = uint32_t(a.B) * uint32_t(a.H), S = uint32_t(a.n_splits);
   uint32_t grp, rank;  // (batch, head) pair; rank within it
-  if (G % 8 == 0) {
+  if (a.spread) {
+    grp = uint32_t(i) / S;
+    rank = uint32_t(i) - grp * S;
+  } else if (G % 8 == 0) {
     const uint32_t g8 = G / 8, slot = uint32_t(i) / 8;
     rank = slot / g8;
     grp = uint32_t(i) % 8 * g8 + (slot - rank * g8);
