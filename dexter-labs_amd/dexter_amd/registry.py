@@ -33,8 +33,8 @@ from typing import Callable, Iterator
 
 from .platform import Capability, PlatformInfo, current_platform
 
-__all__ = ["NoKernelError", "Priority", "KernelSpec", "register", "select", "select_spec", "candidates",
-           "explain", "registered", "unregister"]
+__all__ = ["NoKernelError", "Priority", "KernelSpec", "register", "select", "select_spec",
+           "candidates", "explain", "registered", "unregister"]
 
 PIN_ENV = "DEXTER_KERNEL"
 
